@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -17,6 +18,7 @@
 #include <numeric>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -36,6 +38,7 @@
 #endif
 #include "kernels_dyn.h"
 #include "kernels_tracer.h"
+#include "kernels_ring2.h"
 #include "kernels_limiter.h"
 
 namespace {
@@ -453,6 +456,109 @@ static Patches build_patches(const Topo &t, int P) {
   return pt;
 }
 
+// f(first, last) over [0, n) on up to 8 threads; where no thread can be had the range runs
+// on the caller.  f must not throw.
+template <class F> static void parallel_ranges(int n, F &&f) {
+  const int part = (n + 7) / 8;
+  std::vector<std::thread> th;
+  th.reserve(8);
+  for (int a = 0; a < n; a += part) {
+    const int b = std::min(n, a + part);
+    try {
+      th.emplace_back([&f, a, b] { f(a, b); });
+    } catch (const std::system_error &) {
+      f(a, b);
+    }
+  }
+  for (auto &x : th) x.join();
+}
+
+// Cells, faces and mesh constants of the two-ring stencil (kernels_ring2.h), per column.
+// ok is false where some column's neighbourhood is not the one those kernels hold: npoly
+// 5 or 6 for the column and its neighbours, consecutive slots adjacent, and one common
+// outer neighbour per consecutive pair.
+struct Ring2 {
+  bool ok = true;
+  std::vector<int> cell, face;       // nw x 12, nw x 24
+  std::vector<unsigned> out;         // nw
+  std::vector<int> slot;             // nw x 36: slot in n_j's table per role, -1 if absent
+};
+// roles of n_j's slots seen from the column: the column, n_j-1, n_j+1, mid_j-1, mid_j, far_j
+constexpr int RING2_ROLES = 6;
+
+static Ring2 build_ring2(const Topo &t, const olamgpu_mesh *m) {
+  Ring2 r;
+  r.cell.resize((size_t)t.nw * 12); r.face.assign((size_t)t.nw * 24, 0);
+  r.out.assign(t.nw, 0u); r.slot.assign((size_t)t.nw * 36, -1);
+  for (int c = 0; c < t.nw; ++c)
+    if (t.w_npoly[c] != 5 && t.w_npoly[c] != 6) { r.ok = false; return r; }
+  std::atomic<int> bad{0};
+  parallel_ranges(t.nw, [&](int c0, int c1) {
+    std::atomic<int> *fail = &bad;
+    for (int c = c0; c < c1; ++c) {
+      const int np = t.w_npoly[c];
+      const int *nb = &t.w_nbr[(size_t)c * NSLOT];
+      int *cell = &r.cell[(size_t)c * 12], *face = &r.face[(size_t)c * 24], *slot = &r.slot[(size_t)c * 36];
+      int rest[6][3], nrest[6];
+      for (int i = 0; i < 12; ++i) cell[i] = c;
+      // the column's, the previous and the next ring-1 cell's slot in n_j, and the others
+      for (int j = 0; j < np; ++j) {
+        const int n = nb[j], prev = nb[(j + np - 1) % np], next = nb[(j + 1) % np];
+        int *sl = slot + j * 6;
+        nrest[j] = 0;
+        for (int i = 0; i < t.w_npoly[n]; ++i) {
+          const int x = t.w_nbr[(size_t)n * NSLOT + i];
+          const int role = x == c ? 0 : (x == prev ? 1 : (x == next ? 2 : -1));
+          if (role >= 0) {
+            if (sl[role] >= 0) { *fail = 1; return; }
+            sl[role] = i;
+          } else if (nrest[j] < 3) {
+            rest[j][nrest[j]++] = i;
+          } else { *fail = 1; return; }
+        }
+        if (sl[0] < 0 || sl[1] < 0 || sl[2] < 0) { *fail = 1; return; }
+      }
+      for (int j = 0; j < np; ++j) {
+        const int jn = (j + 1) % np, n = nb[j], o = nb[jn];
+        int found = 0;
+        for (int i = 0; i < nrest[j]; ++i)
+          for (int k = 0; k < nrest[jn]; ++k) {
+            const int x = t.w_nbr[(size_t)n * NSLOT + rest[j][i]];
+            if (x != t.w_nbr[(size_t)o * NSLOT + rest[jn][k]]) continue;
+            ++found;
+            cell[j] = x;
+            slot[j * 6 + 4] = rest[j][i];
+            slot[jn * 6 + 3] = rest[jn][k];
+          }
+        if (found != 1) { *fail = 1; return; }
+      }
+      if (np == 5) cell[5] = cell[4];                 // read through slot 5 for n_0's mid_j-1
+      for (int j = 0; j < np; ++j) {
+        int *sl = slot + j * 6;
+        int extra = 0;
+        for (int i = 0; i < nrest[j]; ++i)
+          if (rest[j][i] != sl[3] && rest[j][i] != sl[4]) { sl[5] = rest[j][i]; ++extra; }
+        if (sl[3] == sl[4] || extra > 1) { *fail = 1; return; }
+        if (sl[5] >= 0) cell[6 + j] = t.w_nbr[(size_t)nb[j] * NSLOT + sl[5]];
+        // faces, and whether a positive flux (from iw1 to iw2) leaves n_j
+        const int role[4] = {2, 3, 4, 5};
+        for (int q = 0; q < 4; ++q) {
+          const int i = sl[role[q]];
+          if (i < 0) continue;
+          face[q * 6 + j] = t.w_face[(size_t)nb[j] * NSLOT + i];
+          if (m->w_dirv[(size_t)(t.perm_w[nb[j]] + 1) * 7 + i] < 0.f) r.out[c] |= 1u << (q * 6 + j);
+        }
+      }
+      if (np == 5) {                                  // slot 5 repeats the face of n_4 and n_0
+        face[5] = face[4];
+        if (r.out[c] & (1u << 4)) r.out[c] |= 1u << 5;
+      }
+    }
+  });
+  r.ok = bad == 0;
+  return r;
+}
+
 // ------------------------------------------------------------------ implementation
 // ---------------------------------------------------------------- allocation-free mass sums
 // olamgpu_mass_sums_noalloc forms the sums of olamgpu_mass_sums with its per-block partial
@@ -639,6 +745,17 @@ struct Impl : ImplBase {
   // at the bench size: it gathers the two-ring stencil of every upwind neighbour).
   bool two_pass = false, fused_fwd = false;
   bool fuse_adj = true;     // one pass for the column and face parts of the adjoint stage
+  // Unlimited stages of orders 2 and 3 and their adjoint as one pass over the two-ring
+  // stencil (kernels_ring2.h), faster at every size measured, from 16,002 columns of 30
+  // levels and one tracer (0.031 against 0.050 ms per stage) to 1,024,002 of 60 and ten
+  // (3.62 against 6.68).  The arrangements above run where it cannot: order 1 (no second
+  // ring), limited final stages (their limiter reads the gradients), columns of more than
+  // 124 levels (two overlapping waves end there), fields of 4 GiB and more (32-bit row
+  // offsets), meshes with other neighbourhoods than pentagons and hexagons, and when one
+  // of them is asked for by name.
+  bool use_ring2 = false;
+  DevBuf b_r2cell, b_r2kf, b_r2face, b_r2out, b_r2ka, b_vr;
+  Ring2Tab<R> r2{};
   // state
   DevBuf thil[2], wmc, wc, vxe, vye, vze, vmc, vc, vmasc, wmasc, alpha, pwfac, pvfac, thilt, vmxet, vmyet, vmzet, vmt;
   DevBuf rho, press, rho_old;
@@ -741,7 +858,72 @@ struct Impl : ImplBase {
       use_patch = two_pass = fused_fwd = false;
       fuse_adj = true;
     }
-    build_patch_tables();
+    if (use_patch) build_patch_tables();
+    use_ring2 = prm.scal_horiz_adv_order >= 2 && ntr > 0 && !(use_patch || two_pass || fused_fwd || !fuse_adj) &&
+                mza <= RING2_TALL_MZA && wsz * sizeof(R) < (size_t(1) << 32);
+    if (use_ring2) build_ring2_tables(m);
+  }
+
+  // Mesh constants of the two-ring stencil: with off_t(m, i) the reconstruction offsets of
+  // cell m at its face i and cof_t(m, i) the weight of its neighbour i in the terms t, the
+  // value that m = n_j gives this column's face reads neighbour i of m with
+  // sum_t off_t(m, back) cof_t(m, i) (kf), and this column enters the value m gives its
+  // face i with sum_t cof_t(m, back) off_t(m, i) (ka).
+  void build_ring2_tables(const olamgpu_mesh *m) {
+    const Ring2 h = build_ring2(t, m);
+    if (!h.ok) { use_ring2 = false; return; }
+    const bool q3 = prm.scal_horiz_adv_order == 3;
+    const int nt = q3 ? 5 : 2;
+    In in{m};
+    const float *offs[5] = {m->v_dxps, m->v_dyps, m->xx0_v, m->xy0_v, m->yy0_v};
+    auto cof = [&](int c, int i, double *o) {
+      const size_t x = (size_t)(t.perm_w[c] + 1) * 7 + i;
+      if (q3) for (int q = 0; q < 5; ++q) o[q] = m->xy_h[x * 5 + q];
+      else { o[0] = m->gxps_coef[x]; o[1] = m->gyps_coef[x]; }
+    };
+    auto off = [&](int c, int i, double *o) {
+      const int oc = t.perm_w[c], v = in.iv(i, oc);
+      const int side = m->w_dirv[(size_t)(oc + 1) * 7 + i] < 0.f ? 0 : 1;
+      for (int q = 0; q < nt; ++q) o[q] = offs[q][(size_t)(v + 1) * 2 + side];
+    };
+    std::vector<R> kf((size_t)nw * 36, R(0)), ka((size_t)nw * 42, R(0));
+    parallel_ranges(nw, [&](int c0, int c1) {
+      for (int c = c0; c < c1; ++c) {
+        const int np = t.w_npoly[c];
+        double cs[5] = {};
+        for (int j = 0; j < np; ++j) {
+          double x[5];
+          cof(c, j, x);
+          for (int q = 0; q < nt; ++q) cs[q] += x[q];
+        }
+        for (int j = 0; j < np; ++j) {
+          const int n = t.w_nbr[(size_t)c * NSLOT + j];
+          const int *sl = &h.slot[(size_t)c * 36 + j * 6];
+          double ob[5], cb[5], oc[5], sum = 0.0;
+          off(n, sl[0], ob);
+          cof(n, sl[0], cb);
+          off(c, j, oc);
+          double own = 1.0;
+          for (int q = 0; q < nt; ++q) own -= cs[q] * oc[q];
+          ka[(size_t)c * 42 + 36 + j] = (R)own;
+          for (int role = 0; role < RING2_ROLES; ++role) {
+            if (sl[role] < 0) continue;
+            double ci[5], oi[5], f = 0.0, a = 0.0;
+            cof(n, sl[role], ci);
+            off(n, sl[role], oi);
+            for (int q = 0; q < nt; ++q) { f += ob[q] * ci[q]; a += cb[q] * oi[q]; }
+            sum += f;
+            if (role > 0) kf[(size_t)c * 36 + j * 6 + role] = (R)f;
+            ka[(size_t)c * 42 + j * 6 + role] = (R)a;
+          }
+          kf[(size_t)c * 36 + j * 6] = (R)sum;
+        }
+      }
+    });
+    upv(b_r2cell, h.cell); upv(b_r2face, h.face); upv(b_r2out, h.out);
+    upv(b_r2kf, kf); upv(b_r2ka, ka);
+    r2.cell = dp<int>(b_r2cell); r2.face = dp<int>(b_r2face); r2.out = dp<unsigned>(b_r2out);
+    r2.kf = dp<R>(b_r2kf); r2.ka = dp<R>(b_r2ka);
   }
 
   // Patches of 8 * cpw columns (one block of 8 waves, cpw owned columns per wave),
@@ -1106,6 +1288,7 @@ struct Impl : ImplBase {
     size_t tb = std::max<size_t>(1, (size_t)ntr) * wsz * sizeof(R);
     for (DevBuf *b : {&adjA, &adjB, &lam0, &nu, &lpart}) { b->alloc(tb); zero(*b); }
     lgG.alloc(2 * tb); zero(lgG);
+    if (use_ring2) b_vr.alloc(wsz * sizeof(R));
     if (prm.scal_horiz_adv_order == 3)
       for (DevBuf &b : lgq) { b.alloc(tb); zero(b); }
     HIPCHK(hipStreamSynchronize(s));
@@ -1594,6 +1777,14 @@ struct Impl : ImplBase {
   // tracers (grad_t2d or grad_t2d_quadratic, scalar_v_column + scalar_w_column)
   void tracer_update(const TrStage<R, RP> &a) {
     // a limited final stage keeps the gradients: the limiter passes read them
+    if (use_ring2 && !a.lim) {
+      const bool q3 = a.order == 3;
+      if (q3 && dm.tall) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, true, true>), dim3(nblk_tr()), dim3(256), dm, r2, a);
+      else if (q3) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, true, false>), dim3(nblk_tr()), dim3(256), dm, r2, a);
+      else if (dm.tall) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, false, true>), dim3(nblk_tr()), dim3(256), dm, r2, a);
+      else LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, false, false>), dim3(nblk_tr()), dim3(256), dm, r2, a);
+      return;
+    }
     if (a.order < 3 && fused_fwd && !a.lim) {
       LAUNCH("k_tr_stage", (k_tr_stage<R, RP>), dim3(nblk_tr()), dim3(256), dm, a);
       return;
@@ -1643,6 +1834,8 @@ struct Impl : ImplBase {
       if (!lsct.p) lsct.alloc(std::max<size_t>(1, ntr) * wsz * sizeof(R));
     }
     RP *rho_tr = tracer_rho();
+    if (use_ring2)
+      LAUNCH("k_tr_vr", (k_tr_vr<R, RP>), dim3((unsigned)((wsz + 255) / 256)), dim3(256), dm, rho_tr, dp<R>(b_vr));
     // lam0 is not cleared: the first adjoint stage (a.first) starts it from zero
     for (int istage = nrk; istage >= 1; --istage) {
       TrAdj<R, RP> a;
@@ -1674,6 +1867,13 @@ struct Impl : ImplBase {
         if (pa.cpw == 4) LAUNCH_SH("k_tr_adj_patch", (k_tr_adj_patch<R, RP, 4>), g, b, pa.lds, dm, a, pa.tab);
         else if (pa.cpw == 2) LAUNCH_SH("k_tr_adj_patch", (k_tr_adj_patch<R, RP, 2>), g, b, pa.lds, dm, a, pa.tab);
         else LAUNCH_SH("k_tr_adj_patch", (k_tr_adj_patch<R, RP, 1>), g, b, pa.lds, dm, a, pa.tab);
+      } else if (use_ring2) {
+        const bool q3 = a.order == 3;
+        const R *vr = dp<R>(b_vr);
+        if (q3 && dm.tall) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, true, true>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
+        else if (q3) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, true, false>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
+        else if (dm.tall) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, false, true>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
+        else LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, false, false>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
       } else {
         adjoint_faces(a);
         adjoint_coefs(a);
