@@ -561,13 +561,10 @@ static Ring2 build_ring2(const Topo &t, const olamgpu_mesh *m) {
 
 // ------------------------------------------------------------------ implementation
 // ---------------------------------------------------------------- allocation-free mass sums
-// olamgpu_mass_sums_noalloc forms the sums of olamgpu_mass_sums with its per-block partial
-// sums in this file-scope device array instead of a buffer the library allocates: a
-// fixed grid of MASS_NB blocks strides over the columns, each block keeping MASS_NV
-// partials (dry mass and up to 64 tracers).  Each GPU holds its own copy of the array
-// until the process ends; every call on a GPU shares it, so calls that overlap on one GPU
-// race.  A call writes every partial it reads, so nothing needs clearing between calls.
-constexpr int MASS_NB = 1024, MASS_NV = 65;
+// olamgpu_mass_sums_noalloc forms the sums of olamgpu_mass_sums with the per-block partial
+// sums in this file-scope device array instead of a buffer of the context.  Each GPU
+// holds its own copy of the array until the process ends; every call on a GPU shares it,
+// so calls that overlap on one GPU race.  A call writes every partial it reads, so nothing needs clearing between calls.
 static __device__ __align__(256) double scratch[MASS_NB * MASS_NV];     // 520 KiB per GPU
 
 // Device address of `scratch` on each device, taken once per device with that device
@@ -585,37 +582,6 @@ static void scratch_setup(int dev) {
 static double *scratch_ptr(int dev) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   return (dev >= 0 && dev < 64) ? g_scratch[dev] : nullptr;
-}
-
-// Partial sums of rho volt and rho volt q_n (FP64) per block over the columns
-// blockIdx.x * WPB + wave, stepping by gridDim.x * WPB; each wave keeps its own row of
-// LDS partials, summed in a fixed order, so the result is deterministic.
-template <class R, class RP>
-__global__ __launch_bounds__(256) void k_mass_partial_gs(DMesh<R> m, const RP *rho, const R *q, int ntr,
-                                                         long tstride, double *part) {
-  __shared__ double sh[WPB][MASS_NV];
-  const int w = threadIdx.x >> 6, lane = lane_id();
-  for (int v = lane; v <= ntr; v += WAVE) sh[w][v] = 0.0;
-  __syncthreads();
-  const int nitem = m.tall ? 2 * m.nw : m.nw;                // a tall column: two waves
-  for (int g = blockIdx.x * WPB + w; g < nitem; g += gridDim.x * WPB) {
-    const int c = m.tall ? g >> 1 : g;
-    const int l = (m.tall ? (g & 1) * WAVE : 0) + lane, k = l + 1;
-    const bool lev = k >= 2 && k <= m.mza;
-    const long ic = (long)c * m.ldk + l;
-    const double mass = lev ? (double)rho[ic] * m.volt[ic] : 0.0;
-    for (int n = -1; n < ntr; ++n) {
-      double v = n < 0 ? mass : (lev ? mass * (double)q[n * tstride + ic] : 0.0);
-      for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s, WAVE);
-      if (lane == 0) sh[w][n + 1] += v;
-    }
-  }
-  __syncthreads();
-  if ((int)threadIdx.x <= ntr) {
-    double s = 0.0;
-    for (int i = 0; i < WPB; ++i) s += sh[i][threadIdx.x];
-    part[(long)blockIdx.x * MASS_NV + threadIdx.x] = s;
-  }
 }
 
 struct ImplBase {
@@ -1277,7 +1243,7 @@ struct Impl : ImplBase {
     }
     ffimp.alloc((size_t)3 * nw * sizeof(R)); zero(ffimp);
     cflmax.alloc(4 * sizeof(unsigned)); nimp.alloc(sizeof(int)); anyimp.alloc(sizeof(int));
-    masspart.alloc((size_t)nblk(nw) * 65 * sizeof(double));
+    masspart.alloc((size_t)MASS_NB * MASS_NV * sizeof(double));
     massout.alloc(65 * sizeof(double));
     mmkeys.alloc(2 * 64 * sizeof(int)); mmout.alloc(2 * 64 * sizeof(float));
     HIPCHK(hipStreamSynchronize(s));
@@ -1908,12 +1874,15 @@ struct Impl : ImplBase {
   }
 
   // -------------------------------------------------------------- diagnostics
+  // per-block partial sums into part, then the sums of all blocks into out (device)
+  void mass_to(double *part, double *out) {
+    const dim3 g(MASS_NB, (unsigned)std::max(1, (ntr + MASS_G - 1) / MASS_G));
+    LAUNCH("k_mass_partial", (k_mass_partial<R, RP>), g, dim3(256), dm, dp<RP>(rho), dp<R>(trS), ntr, tstride, part);
+    LAUNCH("k_mass_final", k_mass_final, dim3(1 + ntr), dim3(256), (const double *)part, MASS_NB, out);
+    HIPCHK(hipGetLastError());
+  }
   void mass_sums(double *out) override {
-    const unsigned nb = nblk(nw);
-    LAUNCH("k_mass_partial", (k_mass_partial<R, RP>), dim3(nb), dim3(256), dm, dp<RP>(rho), dp<R>(trS), ntr, tstride,
-                       masspart.as<double>());
-    LAUNCH("k_mass_final", k_mass_final, dim3(1), dim3(256), masspart.as<double>(), (int)nb, 1 + ntr,
-                       massout.as<double>());
+    mass_to(masspart.as<double>(), massout.as<double>());
     HIPCHK(hipMemcpyAsync(out, massout.p, (1 + ntr) * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
   }
@@ -1922,17 +1891,15 @@ struct Impl : ImplBase {
   void mass_sums_noalloc(double *out_dev, double *scr) override {
     if (1 + ntr > MASS_NV) throw Err(OLAMGPU_EINVAL, "mass_sums_noalloc carries at most 64 tracers");
     if (!scr) throw Err(OLAMGPU_ESTATE, "scratch address not set up on this device");
-    hipLaunchKernelGGL((k_mass_partial_gs<R, RP>), dim3(MASS_NB), dim3(256), 0, s, dm, dp<RP>(rho), dp<R>(trS), ntr,
-                       tstride, scr);
-    hipLaunchKernelGGL(k_mass_final, dim3(1), dim3(256), 0, s, (const double *)scr, MASS_NB, 1 + ntr, out_dev);
-    HIPCHK(hipGetLastError());
+    mass_to(scr, out_dev);
   }
   // tracer_maxmin (check_nans.F90:164-203): out[2n] = max, out[2n+1] = min of tracer n+1
   void tracer_maxmin(float *out) override {
     if (ntr == 0) return;
     LAUNCH("k_maxmin_init", k_maxmin_init, dim3(1), dim3(128), mmkeys.as<int>(), 2 * ntr);
-    LAUNCH("k_tr_maxmin", (k_tr_maxmin<R>), dim3(nblk(nw)), dim3(256), dm, dp<R>(trS), ntr, tstride,
-           mmkeys.as<int>());
+    // 256 blocks a tracer: with 10 tracers 10 waves per SIMD
+    LAUNCH("k_tr_maxmin", (k_tr_maxmin<R>), dim3(std::min(256u, nblk(nw)), (unsigned)ntr), dim3(256), dm, dp<R>(trS),
+           tstride, mmkeys.as<int>());
     LAUNCH("k_maxmin_final", k_maxmin_final, dim3(1), dim3(128), mmkeys.as<int>(), 2 * ntr, mmout.as<float>());
     HIPCHK(hipMemcpyAsync(out, mmout.p, 2 * ntr * sizeof(float), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
