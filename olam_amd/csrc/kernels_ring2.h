@@ -20,25 +20,92 @@
 // column itself with zero constants.  A mesh with any other neighbourhood keeps the
 // gradient and update passes of kernels_tracer.h.
 //
-// What bounds it: the gathers, 19 rows of a column per tracer from L1 and L2 (4.9 KB,
-// 14 TB/s at the size below), with 7 GB of compulsory HBM traffic per stage.  Measured at
-// NXP=320, L=60, 10 tracers, FP32: forward stage 3.62 ms against 2.10 + 4.58 for
-// k_tr_grad and k_tr_update, adjoint stage 4.51 against 5.25 + 3.26 for k_tr_adj01 and
-// k_tr_adj2; NXP=48, L=60, 8 tracers, order 3: 0.075 against 0.108 + 0.261 and 0.083
-// against 0.124 + 0.241; NXP=40, L=30, one FP64 tracer: 0.031 against 0.011 + 0.039.
+// Two forms.  k_tr_ring2 and k_tr_ring2_adj gather the 19 rows of a column per tracer; the
+// requests from L1 to L2 bound them (0.6 of the rows miss L1).  k_tr_ring2s and
+// k_tr_ring2s_adj stage the rows of 16 (12) consecutive columns in LDS, 4 rows a column,
+// and run at the memory's rate per tracer plus the weights once per wave (about 240 and
+// 400 vector instructions).  Measured per stage, forward and adjoint, staged / gathered /
+// as gradient and update passes (k_tr_grad + k_tr_update, k_tr_adj01 + k_tr_adj2):
+// NXP=160, L=60, 10 tracers, FP32: 0.66 / 0.93 / 1.69 and 0.82 / 1.15 / 2.15 ms;
+// NXP=64, L=70, 20 tracers: 0.34 / 0.63 / 1.04 and 0.42 / 0.73 / 1.31 ms;
+// NXP=48, L=60, 8 tracers, order 3: 0.055 / 0.071 / 0.368 and 0.068 / 0.084 / 0.365 ms.
+// Over 40 steps of 8 FP32 tracers on 40,962 columns, <L q, lam> and <q, L^T lam> differ by
+// 2.1e-7 |q||lam| / sqrt(N) rms (4.9e-7 for the gradient and update passes).
 // A cell that is not finite makes its two rings not finite (its weight may be zero).
 #pragma once
 #include "kernels_tracer.h"
 
-// Mesh constants of the two-ring stencil (see ring2_tables in olamgpu.hip).
+// Record of one column: its indices and constants, each in one run of memory.  A wave
+// reads it with one vector load per 64 words, lane i the word i, and broadcasts words with
+// readlane as it needs them; read with scalar loads, a few registers at a time, the record
+// alone cost a wave several memory latencies (0.43 of 0.77 ms at 256,002 columns).
+enum {
+  R2_NBR = 0, R2_CELL = 6, R2_FACE = 18,   // n_j; mid_j, far_j; faces of the column
+  R2_OUTER = 24,                           // faces n_j|n_j+1, n_j|mid_j-1, n_j|mid_j, n_j|far_j
+  R2_OUT = 48,                             // bit i set where outer face i's positive flux leaves n_j
+  R2_NPOLY = 49,
+  R2_PLACE = 50, R2_PLACEA = 55,           // places of the 18 cells and the column among its block's rows, bytes
+  R2_INTS = 60,
+  // forward constants: dirv, then off and cof (nq terms x 6), then kf, per slot j {sum, prev,
+  // next, mid_j-1, mid_j, far_j}
+  R2_DIRV = 0, R2_OFF = 6,
+  // adjoint constants: dirv, then ka, per slot j {c, prev, next, mid_j-1, mid_j, far_j}, then own_j
+  R2_KA = 6, R2_KOWN = 42, R2_NKA = 48
+};
+__host__ __device__ constexpr int r2_cof(int nq) { return R2_OFF + 6 * nq; }
+__host__ __device__ constexpr int r2_kf(int nq) { return R2_OFF + 12 * nq; }
+__host__ __device__ constexpr int r2_nkf(int nq) { return R2_OFF + 12 * nq + 36; }
 template <class R>
 struct Ring2Tab {
-  const int *cell;       // nw x 12: mid_0..mid_5, far_0..far_5
-  const R *kf;           // nw x 36: per slot j {sum, prev, next, mid_j-1, mid_j, far_j}
-  const int *face;       // nw x 24: faces n_j|n_j+1, n_j|mid_j-1, n_j|mid_j, n_j|far_j
-  const unsigned *out;   // nw: bit i set where face i's positive flux leaves n_j
-  const R *ka;           // nw x 42: per slot j {c, prev, next, mid_j-1, mid_j, far_j}, then own_j
+  const int *ints;       // nw x R2_INTS
+  const R *kf, *ka;      // nw x r2_nkf, nw x R2_NKA
 };
+__device__ __forceinline__ float lane_word(float v, int i) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
+__device__ __forceinline__ double lane_word(double v, int i) {
+  const long long w = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)w, i),
+                 hi = (unsigned)__builtin_amdgcn_readlane((int)(w >> 32), i);
+  return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+struct RecI {
+  int v;
+  __device__ __forceinline__ explicit RecI(const int *t, int c) {
+    const int lane = lane_id();
+    v = lane < R2_INTS ? t[(long)c * R2_INTS + lane] : 0;
+  }
+  __device__ __forceinline__ int operator[](int i) const { return __builtin_amdgcn_readlane(v, i); }
+};
+template <class R, int N>
+struct RecK {
+  static constexpr int NV = (N + WAVE - 1) / WAVE;
+  R v[NV];
+  __device__ __forceinline__ RecK(const R *t, int c) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int x = i * WAVE + lane_id();
+      v[i] = x < N ? t[(long)c * N + x] : R(0);
+    }
+  }
+  __device__ __forceinline__ R operator[](int i) const { return lane_word(v[i / WAVE], i % WAVE); }
+};
+
+// shdn(v, 1) and shup(v, 1) with zero in the lane that has no source, in the form that the
+// compiler folds into the instruction using it.
+template <int CTRL>
+__device__ __forceinline__ float dpp0(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp0(double v) {
+  const long long w = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w, CTRL, 0xF, 0xF, true),
+                 hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(w >> 32), CTRL, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+template <class R> __device__ __forceinline__ R above0(R v) { return dpp0<0x130>(v); }
+template <class R> __device__ __forceinline__ R below0(R v) { return dpp0<0x138>(v); }
 
 // Rows of one tracer field read through a buffer resource: the lane's byte offset in a
 // vector register, the column's in a scalar one, so a gather costs no address arithmetic.
@@ -59,92 +126,184 @@ struct Rows {
 };
 constexpr int ROWS_NT = 2;   // non-temporal: rows read once
 
+template <class R>
+__device__ __forceinline__ unsigned field_bytes(const DMesh<R> &m) {
+  return (unsigned)((size_t)m.nw * m.ldk * sizeof(R));
+}
+
 // Position of a wave: column, tracers and level.  A tall column's two waves overlap by
 // four levels (the first holds levels 1..64 and stores 1..62, the second holds 61..124
 // and stores from 63), so the vertical stencil, two levels each way, needs no exchange
-// between them; columns of more than 124 levels keep the other passes.
+// between them; columns of more than 124 levels keep the other passes.  blockIdx.y is the
+// tracer group, so every wave of a block runs the same number of tracers.  Waves past the
+// last column repeat it and store nothing.
 constexpr int RING2_TALL_BASE = 60, RING2_TALL_MZA = RING2_TALL_BASE + WAVE;
-struct RingItem { int c, n0, n1, l; bool own; };
-template <bool TALL>
+struct RingItem { int b, c, n0, n1, l; bool own; };
+template <bool TALL, int NW>
 __device__ __forceinline__ RingItem ring_item(int nw, int ntr, int tpw) {
-  const TrItem t = tr_item(nw, ntr, tpw, TALL ? 1 : 0);
   RingItem r;
-  r.c = t.c; r.n0 = t.n0; r.n1 = t.n1;
+  r.b = xcd_block(blockIdx.x, gridDim.x);
+  const int w = __builtin_amdgcn_readfirstlane(r.b * NW + (threadIdx.x >> 6));
+  const int lane = lane_id();
+  r.n0 = blockIdx.y * tpw;
+  r.n1 = min(ntr, r.n0 + tpw);
+  r.c = TALL ? w >> 1 : w;
+  r.l = lane;
+  r.own = r.c < nw;
   if constexpr (TALL) {
-    const int lane = lane_id();
-    const bool upper = t.l >= WAVE;
-    r.l = upper ? RING2_TALL_BASE + lane : lane;
-    r.own = upper ? lane >= 2 : lane < RING2_TALL_BASE + 2;
-  } else {
-    r.l = t.l;
-    r.own = true;
+    const bool upper = w & 1;
+    if (upper) r.l = RING2_TALL_BASE + lane;
+    r.own = r.own && (upper ? lane >= 2 : lane < RING2_TALL_BASE + 2);
   }
+  r.c = min(r.c, nw - 1);
   return r;
 }
 
-template <class R, class RP, bool Q3, bool TALL>
-__global__ __launch_bounds__(256) void k_tr_ring2(DMesh<R> m, Ring2Tab<R> t, TrStage<R, RP> a) {
-  const RingItem ti = ring_item<TALL>(m.nw, a.ntr, a.tpw);
-  const int c = ti.c;
-  if (c >= m.nw) return;
-  const int l = ti.l, k = l + 1, mza = m.mza;
-  const unsigned ul = (unsigned)l;
-  const bool act = k <= mza, body = act && k >= 2, inner = k >= 2 && k <= mza - 1;
+// Staging of a tracer's rows in LDS.  The 16 consecutive columns of a forward block (8
+// tall ones) have about 64 cells in their rings (45) where their waves would gather 19 rows
+// each: the block reads every row once, 16 bytes a lane, one tracer ahead of the one it
+// computes from the other of two buffers, one barrier per tracer.  A row keeps the levels
+// in use only, so what lies above them in a lane's read is the next row's.
+constexpr int RING2_NWF = 16, RING2_NWA = 12;      // waves of a staged block, forward and adjoint
+struct Ring2Stage {
+  const int *count;      // per block: rows staged
+  const int *cells;      // blocks x nmax: their columns
+  int nmax;
+  unsigned pitch, magic; // bytes of a row (a multiple of 16), 2^32 / pitch rounded up
+  unsigned bytes;        // of one buffer
+};
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+template <class R, int NCH, int NW>
+struct Stager {
+  unsigned to, from[NCH];
+  bool get_[NCH];
+  u32x4 v[NCH];
+  __device__ __forceinline__ Stager(const Ring2Stage &t, int b, int ldk) {
+    const unsigned total = (unsigned)t.count[b] * t.pitch;
+    to = threadIdx.x * 16u;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const unsigned at = to + (unsigned)(i * NW) * 1024u, cell = __umulhi(at, t.magic);
+      get_[i] = at < total;
+      from[i] = get_[i] ? (unsigned)t.cells[b * t.nmax + (int)cell] * (unsigned)(ldk * sizeof(R)) + (at - cell * t.pitch)
+                        : 0u;
+      v[i] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  __device__ __forceinline__ void get(const Rows<R> &q) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (get_[i]) v[i] = __builtin_amdgcn_raw_buffer_load_b128(q.rs, (int)from[i], 0, 0);
+  }
+  __device__ __forceinline__ void put(unsigned char *buf) const {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (get_[i]) *reinterpret_cast<u32x4 *>(buf + to + (unsigned)(i * NW) * 1024u) = v[i];
+  }
+};
+template <class R>
+__device__ __forceinline__ R lds_row(const unsigned char *buf, unsigned off) {
+  return *reinterpret_cast<const R *>(buf + off);
+}
+
+// Weights of one column for the forward stage (see the head of this file), and what the
+// vertical part and the update need of the column.
+template <class R>
+struct RingFwd {
+  R C[18], S, v0, v1, v2, wf, vt, rinv;
+};
+template <class R, class RP, bool Q3>
+__device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const RecK<R, r2_nkf(Q3 ? 5 : 2)> &K,
+                                         const TrStage<R, RP> &a, int c, int l, RingFwd<R> &f) {
+  const int k = l + 1, mza = m.mza;
+  const bool body = k <= mza && k >= 2, inner = k >= 2 && k <= mza - 1;
   const long ldk = m.ldk, cb = (long)c * ldk;
+  const unsigned rowb = (unsigned)(ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 own = (unsigned)c * rowb;
+  const Rows<R> vr(a.vmasc, (unsigned)m.nv * rowb);
   constexpr int NQ = Q3 ? 5 : 2;
-  const R *off[5] = {m.w_dxs, m.w_dys, m.w_os[0][0], m.w_os[0][1], m.w_os[0][2]};
-  const R *cof[5] = {Q3 ? m.w_q[0][0] : m.w_gxc, Q3 ? m.w_q[0][1] : m.w_gyc, m.w_q[0][2], m.w_q[0][3], m.w_q[0][4]};
-  // weights: w_j is the inflow through face j, taken from n_j; the outflow carries this
-  // column's own reconstruction, whose terms sum to b
+  constexpr int KF = r2_kf(NQ), COF = r2_cof(NQ);
+  // w_j is the inflow through face j, taken from n_j; the outflow carries this column's
+  // own reconstruction, whose terms sum to b
   R w[6], b[NQ], S = R(0);
-  unsigned row[18];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) b[q] = R(0);
+  R vm[6];
+#pragma unroll
+  for (int j = 0; j < 6; ++j) vm[j] = vr.get(lb, (unsigned)I[R2_FACE + j] * rowb);
+  const R wm = Rows<R>(a.wmasc, fb).get(lb, own);
+  const R rf = (R)a.rho[cb + l];
+  f.vt = Rows<R>(m.volti, fb).get(lb, own);
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
-    const int s = c * NSLOT + j;
-    row[j] = (unsigned)m.w_nbr[s] * (unsigned)(ldk * sizeof(R));
-    const R f = m.w_dirv[s] * ldl(a.vmasc + (long)m.w_face[s] * ldk, ul);
-    w[j] = f > R(0) ? f : R(0);
-    const R o = f - w[j];
-    S = S + f;
+    const R x = K[R2_DIRV + j] * vm[j];
+    w[j] = x > R(0) ? x : R(0);
+    const R o = x - w[j];
+    S = S + x;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) b[q] = b[q] + off[q][s] * o;
+    for (int q = 0; q < NQ; ++q) b[q] = b[q] + K[R2_OFF + 6 * q + j] * o;
   }
-#pragma unroll
-  for (int i = 0; i < 12; ++i) row[6 + i] = (unsigned)t.cell[c * 12 + i] * (unsigned)(ldk * sizeof(R));
-  R C[18];
-  const R *kf = t.kf + (long)c * 36;
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     const int jm = (j + 5) % 6, jp = (j + 1) % 6;
     R e = w[j];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) e = e + b[q] * cof[q][c * NSLOT + j];
-    C[j] = e - w[j] * kf[6 * j] + w[jm] * kf[6 * jm + 2] + w[jp] * kf[6 * jp + 1];
-    C[6 + j] = w[j] * kf[6 * j + 4] + w[jp] * kf[6 * jp + 3];
-    C[12 + j] = w[j] * kf[6 * j + 5];
+    for (int q = 0; q < NQ; ++q) e = e + b[q] * K[COF + 6 * q + j];
+    f.C[j] = e - w[j] * K[KF + 6 * j] + w[jm] * K[KF + 6 * jm + 2] + w[jp] * K[KF + 6 * jp + 1];
+    f.C[6 + j] = w[j] * K[KF + 6 * j + 4] + w[jp] * K[KF + 6 * jp + 3];
+    f.C[12 + j] = w[j] * K[KF + 6 * j + 5];
   }
-  if (m.w_npoly[c] == 5) {        // n_4 and n_0 are neighbours; slot 5 reads the column itself
-    C[0] = C[0] + w[4] * kf[6 * 4 + 2];
-    C[4] = C[4] + w[0] * kf[1];
+  if (I[R2_NPOLY] == 5) {         // n_4 and n_0 are neighbours; slot 5 reads the column itself
+    f.C[0] = f.C[0] + w[4] * K[KF + 6 * 4 + 2];
+    f.C[4] = f.C[4] + w[0] * K[KF + 1];
   }
   // vertical: with d(k) = q(k+1) - q(k) on levels 2..mza-1 the upwinded value at W level k
   // less q(k) is v0 d(k-1) + v1 d(k) + v2 d(k+1) (grad_z_quadratic, bounded)
-  const R wm = ldl(a.wmasc + cb, ul);
   const R fexpl = R(1) - a.ffimp[(long)(a.istage - 1) * m.nw + c];
-  const R wf = inner ? fexpl * wm : R(0);
+  f.wf = inner ? fexpl * wm : R(0);
   const int lp = min(l + 1, (int)ldk - 1);
   const bool neg = wm < R(0);
-  const R v0 = neg ? R(0) : wf * m.aw22[l];
-  const R v1 = neg ? wf * (R(1) + m.aw21[lp]) : wf * m.aw12[l];
-  const R v2 = neg ? wf * m.aw11[lp] : R(0);
-  S = S + fexpl * (shup(wm, 1) - wm);
-  const R rf = (R)a.rho[cb + l];
-  const R rinv = R(1) / (body ? rf : R(1));
-  const R vt = ldl(m.volti + cb, ul);
-  const unsigned fb = (unsigned)((size_t)m.nw * ldk * sizeof(R)), lb = ul * (unsigned)sizeof(R),
-                 own = (unsigned)c * (unsigned)(ldk * sizeof(R));
+  f.v0 = neg ? R(0) : f.wf * m.aw22[l];
+  f.v1 = neg ? f.wf * (R(1) + m.aw21[lp]) : f.wf * m.aw12[l];
+  f.v2 = neg ? f.wf * m.aw11[lp] : R(0);
+  f.S = S + fexpl * (below0(wm) - wm);
+  f.rinv = R(1) / (body ? rf : R(1));
+}
+// The new value from the column's value, scp0, tendency and the 18 cells' values; qn(i)
+// is called once per cell.
+template <class R, class F>
+__device__ __forceinline__ R ring_fwd_value(const RingFwd<R> &f, R qc, R q0, R st, R dtr, bool inner, int k, F &&qn) {
+  R d = above0(qc) - qc;
+  d = inner ? d : R(0);
+  const R y = f.v0 * below0(d) + f.v1 * d + f.v2 * above0(d);
+  const R x = y - f.wf * d;                     // the same flux against the level above
+  R F0 = (qc - q0) * f.S + (below0(x) - y), F1 = R(0);
+#pragma unroll
+  for (int i = 0; i < 18; i += 2) {
+    F0 = F0 + f.C[i] * (qn(i) - qc);
+    F1 = F1 + f.C[i + 1] * (qn(i + 1) - qc);
+  }
+  F0 = F0 + F1;
+  R r = q0 + dtr * (st + f.vt * F0) * f.rinv;
+  const R lev1 = above0(r);                     // level 1 copies level 2
+  return k == 1 ? lev1 : r;
+}
+
+template <class R, class RP, bool Q3, bool TALL>
+__global__ __launch_bounds__(256) void k_tr_ring2(DMesh<R> m, Ring2Tab<R> t, TrStage<R, RP> a) {
+  const RingItem ti = ring_item<TALL, WPB>(m.nw, a.ntr, a.tpw);
+  const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
+  const bool inner = k >= 2 && k <= mza - 1;
+  const long cb = (long)c * m.ldk;
+  const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 own = (unsigned)c * rowb;
+  const RecI I(t.ints, c);
+  const RecK<R, r2_nkf(Q3 ? 5 : 2)> K(t.kf, c);
+  RingFwd<R> f;
+  ring_fwd<R, RP, Q3>(m, I, K, a, c, l, f);
+  unsigned row[18];
+#pragma unroll
+  for (int i = 0; i < 18; ++i) row[i] = (unsigned)I[R2_NBR + i] * rowb;
   const bool start = a.q_in == a.q0;
   for (int n = ti.n0; n < ti.n1; ++n) {
     const long fo = n * a.tstride;
@@ -155,17 +314,52 @@ __global__ __launch_bounds__(256) void k_tr_ring2(DMesh<R> m, Ring2Tab<R> t, TrS
     for (int i = 0; i < 18; ++i) qn[i] = q.get(lb, row[i]);
     const R q0 = start ? qc : Rows<R>(a.q0 + fo, fb).template get<ROWS_NT>(lb, own);
     const R st = a.sct ? Rows<R>(a.sct + fo, fb).template get<ROWS_NT>(lb, own) : R(0);
-    R d = shdn(qc, 1) - qc;
-    d = inner ? d : R(0);
-    const R y = v0 * shup(d, 1) + v1 * d + v2 * shdn(d, 1);
-    const R x = y - wf * d;                     // the same flux against the level above
-    R F = (qc - q0) * S + (shup(x, 1) - y);
+    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, k, [&](int i) { return qn[i]; });
+    if (k <= mza && ti.own) st_nt(a.q_out + fo, cb + l, r);
+  }
+}
+
+template <class R, class RP, bool Q3, bool TALL, int NCH>
+__global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_tr_ring2s(DMesh<R> m, Ring2Tab<R> t, Ring2Stage sg,
+                                                               TrStage<R, RP> a) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const RingItem ti = ring_item<TALL, RING2_NWF>(m.nw, a.ntr, a.tpw);
+  const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
+  const bool inner = k >= 2 && k <= mza - 1;
+  const long cb = (long)c * m.ldk;
+  const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 own = (unsigned)c * rowb;
+  const RecI I(t.ints, c);
+  const RecK<R, r2_nkf(Q3 ? 5 : 2)> K(t.kf, c);
+  Stager<R, NCH, RING2_NWF> st_(sg, ti.b, m.ldk);
+  const bool start = a.q_in == a.q0;
+  R q0n = R(0), stn = R(0);
+  auto fetch = [&](int n) {
+    const long fo = n * a.tstride;
+    st_.get(Rows<R>(a.q_in + fo, fb));
+    if (!start) q0n = Rows<R>(a.q0 + fo, fb).template get<ROWS_NT>(lb, own);
+    if (a.sct) stn = Rows<R>(a.sct + fo, fb).template get<ROWS_NT>(lb, own);
+  };
+  fetch(ti.n0);
+  RingFwd<R> f;
+  ring_fwd<R, RP, Q3>(m, I, K, a, c, l, f);
+  unsigned row[19];
 #pragma unroll
-    for (int i = 0; i < 18; ++i) F = F + C[i] * (qn[i] - qc);
-    R r = q0 + a.dtr * (st + vt * F) * rinv;
-    const R lev1 = shdn(r, 1);                  // level 1 copies level 2
-    if (k == 1) r = lev1;
-    if (act && ti.own) st_nt(a.q_out + fo, cb + l, r);
+  for (int i = 0; i < 19; ++i) row[i] = (((unsigned)I[R2_PLACE + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch;
+  st_.put(smem_raw);
+  __syncthreads();
+  for (int n = ti.n0; n < ti.n1; ++n) {
+    const unsigned char *buf = smem_raw + ((n - ti.n0) & 1) * sg.bytes + lb;
+    const R qc = lds_row<R>(buf, row[18]);
+    const R q0 = start ? qc : q0n, st = stn;
+    const bool more = n + 1 < ti.n1;
+    if (more) fetch(n + 1);
+    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, k, [&](int i) { return lds_row<R>(buf, row[i]); });
+    if (k <= mza && ti.own) st_nt(a.q_out + n * a.tstride, cb + l, r);
+    if (more) {
+      st_.put(smem_raw + ((n + 1 - ti.n0) & 1) * sg.bytes);
+      __syncthreads();
+    }
   }
 }
 
@@ -185,43 +379,59 @@ __global__ __launch_bounds__(256) void k_tr_vr(DMesh<R> m, const RP *rho, R *out
 // cells m, through m's reconstruction coefficient that points back here.  Lane 0 carries
 // level 2's weights, so what mu holds at level 1 (a copy of level 2 in the forward stage)
 // is weighted as level 2 and then added there.
-template <class R, class RP, bool Q3, bool TALL>
-__global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t, TrAdj<R, RP> a, const R *vr) {
-  const RingItem ti = ring_item<TALL>(m.nw, a.ntr, a.tpw);
-  const int c = ti.c;
-  if (c >= m.nw) return;
-  const int l = ti.l, k = l + 1, mza = m.mza;
-  const unsigned ul = (unsigned)l, um = ul ? ul : 1u;
-  const bool act = k <= mza, body = act && k >= 2, inner = k >= 2 && k <= mza - 1;
-  const long ldk = m.ldk, cb = (long)c * ldk;
-  R D[18];
-  unsigned row[18];
+//
+// With no implicit column and no limited stage (on) the scp0 terms need no array of their
+// own: the buffers of the earlier stages' mu are still there, and the last stage adds
+// mu_s - nu_s cc of every stage s to lq, smallest first, so the result is rounded once at
+// its own size instead of once per stage.
+template <class R>
+struct AdjHist {
+  int on;
+  const R *mu3, *mu2;    // mu of the final stage (the adjoint at entry) and, in RK3, of stage 2
+  R dt3, dt2;            // their time steps
+};
+template <class R>
+struct RingAdj {
+  R D[18], Dc, g, gc, cc, wf, al, be, cm, c0, cp;
+  bool rd0;
+};
+// vr(i): volti / rho of cell i (18: this column) at the lane's weight level
+template <class R, class RP, class F>
+__device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const RecK<R, R2_NKA> &K,
+                                         const TrAdj<R, RP> &a, int c, int l, RingAdj<R> &f, F &&vr) {
+  const int k = l + 1, mza = m.mza;
+  const bool body = k <= mza && k >= 2, inner = k >= 2 && k <= mza - 1;
+  const long ldk = m.ldk;
+  const unsigned rowb = (unsigned)(ldk * sizeof(R)), lb = (unsigned)l * (unsigned)sizeof(R),
+                 mb = (l ? (unsigned)l : 1u) * (unsigned)sizeof(R);
+  const Rows<R> vf(a.vmasc, (unsigned)m.nv * rowb);
+  R *D = f.D;
 #pragma unroll
   for (int i = 0; i < 18; ++i) D[i] = R(0);
-  const R *ka = t.ka + (long)c * 42;
-  const int *f2 = t.face + (long)c * 24;
-  const unsigned out = t.out[c];
-  auto flux = [&](int i) {       // outflow of n_j positive
-    const R v = ldl(a.vmasc + (long)f2[i] * ldk, um);
-    return ((out >> i) & 1u) ? v : -v;
-  };
-  auto pos = [](R v) { return v > R(0) ? v : R(0); };
-  R csum = R(0), rim[6], fix0 = R(0), fix4 = R(0);
+  // every flux first, then the weights
+  R vm[6], vo[24];
 #pragma unroll
-  for (int j = 0; j < 6; ++j) rim[j] = flux(j);
+  for (int j = 0; j < 6; ++j) vm[j] = vf.get(mb, (unsigned)I[R2_FACE + j] * rowb);
+#pragma unroll
+  for (int i = 0; i < 24; ++i) vo[i] = vf.get(mb, (unsigned)I[R2_OUTER + i] * rowb);
+  const unsigned out = (unsigned)I[R2_OUT];
+#pragma unroll
+  for (int i = 0; i < 24; ++i) vo[i] = vo[i] * (((out >> i) & 1u) ? R(1) : R(-1));     // outflow of n_j positive
+  const R wm = Rows<R>(a.wmasc, field_bytes(m)).get(lb, (unsigned)c * rowb);
+  auto pos = [](R v) { return v > R(0) ? v : R(0); };
+  R csum = R(0), fix0 = R(0), fix4 = R(0);
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
-    const int s = c * NSLOT + j, jm = (j + 5) % 6, jp = (j + 1) % 6;
-    row[j] = (unsigned)m.w_nbr[s] * (unsigned)(ldk * sizeof(R));
-    const R f = m.w_dirv[s] * ldl(a.vmasc + (long)m.w_face[s] * ldk, um);
-    csum = csum + f;
-    const R in = pos(f);
-    R sum = ka[6 * j] * in;
-    const R tp = ka[6 * j + 1] * pos(-rim[jm]), tn = ka[6 * j + 2] * pos(rim[j]);
-    const R tmp_ = ka[6 * j + 3] * pos(flux(6 + j)), tmn = ka[6 * j + 4] * pos(flux(12 + j)),
-            tf = ka[6 * j + 5] * pos(flux(18 + j));
+    const int jm = (j + 5) % 6, jp = (j + 1) % 6;
+    const R x = K[R2_DIRV + j] * vm[j];
+    csum = csum + x;
+    const R in = pos(x);
+    R sum = K[R2_KA + 6 * j] * in;
+    const R tp = K[R2_KA + 6 * j + 1] * pos(-vo[jm]), tn = K[R2_KA + 6 * j + 2] * pos(vo[j]);
+    const R tmp_ = K[R2_KA + 6 * j + 3] * pos(vo[6 + j]), tmn = K[R2_KA + 6 * j + 4] * pos(vo[12 + j]),
+            tf = K[R2_KA + 6 * j + 5] * pos(vo[18 + j]);
     sum = sum + tp + tn + tmp_ + tmn + tf;
-    D[j] = D[j] + ka[36 + j] * (in - f) - sum;
+    D[j] = D[j] + K[R2_KOWN + j] * (in - x) - sum;
     D[jm] = D[jm] + tp;
     D[jp] = D[jp] + tn;
     if (j == 0) fix4 = tp;
@@ -230,65 +440,177 @@ __global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t,
     D[6 + j] = D[6 + j] + tmn;
     D[12 + j] = tf;
   }
-  if (m.w_npoly[c] == 5) {        // n_4 and n_0 are neighbours, slot 5 is the column itself
+  if (I[R2_NPOLY] == 5) {         // n_4 and n_0 are neighbours, slot 5 is the column itself
     D[0] = D[0] + fix0;
     D[4] = D[4] + fix4;
     D[5] = R(0);
   }
+  // the weights of a column sum to zero; its own is summed ring by ring from the smallest
+  // terms on (far, mid, ring 1), not one rounding after another at the size of the sum
+  auto six = [&](int b) { return ((D[b] + D[b + 3]) + (D[b + 1] + D[b + 4])) + (D[b + 2] + D[b + 5]); };
+  const R Dc = -((six(12) + six(6)) + six(0));
 #pragma unroll
-  for (int i = 0; i < 12; ++i) row[6 + i] = (unsigned)t.cell[c * 12 + i] * (unsigned)(ldk * sizeof(R));
-  R Dc = R(0);
-  const unsigned fb = (unsigned)((size_t)m.nw * ldk * sizeof(R)), lb = ul * (unsigned)sizeof(R),
-                 mb = um * (unsigned)sizeof(R), own = (unsigned)c * (unsigned)(ldk * sizeof(R));
-  const Rows<R> gr(vr, fb);
-#pragma unroll
-  for (int i = 0; i < 18; ++i) {
-    Dc = Dc - D[i];
-    D[i] = D[i] * (a.dtr * gr.get(mb, row[i]));
-  }
-  const R g = a.dtr * gr.get(mb, own);
-  Dc = Dc * g;
+  for (int i = 0; i < 18; ++i) D[i] = D[i] * vr(i);
+  const R gc = vr(18);
+  f.gc = body ? gc : R(0);
+  f.g = a.dtr * f.gc;
+  f.Dc = Dc * gc;
   // vertical transpose: upw(k) feeds F(k+1) with +wf and F(k) with -wf
-  const R wm = ldl(a.wmasc + cb, ul);
   const R ff = a.ffimp[(long)(a.istage - 1) * m.nw + c];
   const R fexpl = R(1) - ff;
-  const R cc = csum + fexpl * (shup(wm, 1) - wm);
-  const R wf = inner ? fexpl * wm : R(0);
+  f.cc = csum + fexpl * (below0(wm) - wm);
+  f.wf = inner ? fexpl * wm : R(0);
   const bool neg = wm < R(0);
   const bool neg_m1 = shup((int)neg, 1) != 0, neg_p1 = shdn((int)neg, 1) != 0;
   const int lp = min(l + 1, (int)ldk - 1);
-  const R al = (inner && !neg) ? R(1) : R(0), be = (body && k >= 3 && neg_m1) ? R(1) : R(0);
-  const R cm = (inner && k >= 3 && neg_m1) ? m.aw11[l] : R(0);
-  const R c0 = inner ? (neg ? m.aw21[lp] : m.aw12[l]) : R(0);
-  const R cp = (k >= 2 && k <= mza - 2 && !neg_p1) ? m.aw22[lp] : R(0);
+  f.al = (inner && !neg) ? R(1) : R(0);
+  f.be = (body && k >= 3 && neg_m1) ? R(1) : R(0);
+  f.cm = (inner && k >= 3 && neg_m1) ? m.aw11[l] : R(0);
+  f.c0 = inner ? (neg ? m.aw21[lp] : m.aw12[l]) : R(0);
+  f.cp = (k >= 2 && k <= mza - 2 && !neg_p1) ? m.aw22[lp] : R(0);
   // on the first adjoint stage lam0 holds only what the implicit pass of this column wrote
-  const bool rd0 = !a.first || ff > R(0.001);
+  f.rd0 = !a.first || ff > R(0.001);
+}
+// what mu holds at level 1 counts as level 2's
+template <class R>
+__device__ __forceinline__ R ring_fold(R mr, bool body, int k) {
+  const R below = below0(mr);
+  return body ? (k == 2 ? mr + below : mr) : R(0);
+}
+// lq from the column's mu and its cells', and the stage's scp0 terms
+template <class R, class F>
+__device__ __forceinline__ R ring_adj_value(const RingAdj<R> &f, R mr, R &mu, R &nucc, R dtr, bool body, int k,
+                                            F &&mn) {
+  mu = ring_fold(mr, body, k);
+  const R nu = mu * f.g;
+  nucc = nu * f.cc;
+  const R L = f.wf * (above0(nu) - nu);
+  const R Lm = below0(L);
+  const R lds = f.cm * Lm + f.c0 * L + f.cp * above0(L);
+  R acc = f.Dc * mr, acb = R(0);
+#pragma unroll
+  for (int i = 0; i < 18; i += 2) {
+    acc = acc + f.D[i] * mn(i);
+    acb = acb + f.D[i + 1] * mn(i + 1);
+  }
+  acc = acc + acb;
+  const R acc1 = below0(acc);
+  if (k == 2) acc = acc + acc1;
+  const R lq = dtr * acc + (f.al * L + f.be * Lm + (below0(lds) - lds));
+  return body ? lq : R(0);
+}
+
+// The own-column rows a stage reads besides mu: lam0, or at the last stage of an AdjHist
+// the earlier stages' mu
+template <class R, class RP>
+__device__ __forceinline__ void ring_adj_rows(const TrAdj<R, RP> &a, const AdjHist<R> &h, bool rd0, const R *&p1,
+                                              const R *&p2) {
+  p1 = h.on ? (a.last ? h.mu3 : nullptr) : (rd0 ? a.lam0 : nullptr);
+  p2 = h.on && a.last ? h.mu2 : nullptr;
+}
+template <class R, class RP>
+__device__ __forceinline__ void ring_adj_store(const TrAdj<R, RP> &a, const AdjHist<R> &h, const RingAdj<R> &f, R lq,
+                                               R mu, R nucc, R p, R q, bool body, int k, bool st, int n, long i) {
+  const long fo = n * a.tstride;
+  R r = lq;
+  if (h.on) {
+    if (a.last) {               // stage 1 read q = scp0
+      const R mu3 = ring_fold(p, body, k), mu2 = ring_fold(q, body, k);
+      const R s = (lq + (mu - nucc)) + (mu2 - f.cc * (f.gc * (h.dt2 * mu2 + h.dt3 * mu3)));
+      r = body ? mu3 + s : R(0);
+    }
+  } else {
+    const R l0 = body ? p + mu - nucc : p;
+    if (a.last) r = lq + l0;
+    else if (st) st_nt(a.lam0 + fo, i, l0);
+  }
+  if (st) st_nt(a.lq + fo, i, r);
+}
+
+template <class R, class RP, bool TALL>
+__global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t, TrAdj<R, RP> a, AdjHist<R> h,
+                                                      const R *vr) {
+  const RingItem ti = ring_item<TALL, WPB>(m.nw, a.ntr, a.tpw);
+  const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
+  const bool act = k <= mza, body = act && k >= 2;
+  const long cb = (long)c * m.ldk;
+  const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 mb = (l ? (unsigned)l : 1u) * (unsigned)sizeof(R);
+  const RecI I(t.ints, c);
+  const RecK<R, R2_NKA> K(t.ka, c);
+  unsigned row[19];
+#pragma unroll
+  for (int i = 0; i < 18; ++i) row[i] = (unsigned)I[R2_NBR + i] * rowb;
+  row[18] = (unsigned)c * rowb;
+  const Rows<R> gr(vr, fb);
+  RingAdj<R> f;
+  ring_adj(m, I, K, a, c, l, f, [&](int i) { return gr.get(mb, row[i]); });
+  const R *p1, *p2;
+  ring_adj_rows(a, h, f.rd0, p1, p2);
   for (int n = ti.n0; n < ti.n1; ++n) {
     const long fo = n * a.tstride;
     const Rows<R> q(a.mu + fo, fb);
-    const R mr = q.get(lb, own);
+    const R mr = q.get(lb, row[18]);
     R mn[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) mn[i] = q.get(lb, row[i]);
-    R l0 = rd0 ? Rows<R>(a.lam0 + fo, fb).template get<ROWS_NT>(lb, own) : R(0);
-    const R below = shup(mr, 1);
-    const R mu = k == 1 ? R(0) : (k == 2 ? mr + below : mr);
-    const R nu = mu * g;
-    if (body) l0 = l0 + mu - nu * cc;
-    const R L = wf * (shdn(nu, 1) - nu);
-    const R Lm = shup(L, 1);
-    const R lds = cm * Lm + c0 * L + cp * shdn(L, 1);
-    R acc = Dc * mr;
+    const R p = p1 ? Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
+    const R q2 = p2 ? Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
+    R mu, nucc;
+    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i) { return mn[i]; });
+    ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
+  }
+}
+
+template <class R, class RP, bool TALL, int NCH>
+__global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr_ring2s_adj(DMesh<R> m, Ring2Tab<R> t, Ring2Stage sg,
+                                                                   TrAdj<R, RP> a, AdjHist<R> h, const R *vr) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const RingItem ti = ring_item<TALL, RING2_NWA>(m.nw, a.ntr, a.tpw);
+  const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
+  const bool act = k <= mza, body = act && k >= 2;
+  const long cb = (long)c * m.ldk;
+  const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 mb = (l ? (unsigned)l : 1u) * (unsigned)sizeof(R), own = (unsigned)c * rowb;
+  const RecI I(t.ints, c);
+  const RecK<R, R2_NKA> K(t.ka, c);
+  Stager<R, NCH, RING2_NWA> st_(sg, ti.b, m.ldk);
+  const bool rd0 = !a.first || a.ffimp[(long)(a.istage - 1) * m.nw + c] > R(0.001);
+  const R *p1, *p2;
+  ring_adj_rows(a, h, rd0, p1, p2);
+  R pn = R(0), qn = R(0);
+  auto fetch = [&](int n) {
+    const long fo = n * a.tstride;
+    st_.get(Rows<R>(a.mu + fo, fb));
+    if (p1) pn = Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, own);
+    if (p2) qn = Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, own);
+  };
+  // vr goes where the second tracer will be; with it the first tracer, so that the
+  // weights are formed with no rows in flight
+  Stager<R, NCH, RING2_NWA> sv(st_);
+  sv.get(Rows<R>(vr, fb));
+  fetch(ti.n0);
+  sv.put(smem_raw + sg.bytes);
+  st_.put(smem_raw);
+  __syncthreads();
+  unsigned row[19];
 #pragma unroll
-    for (int i = 0; i < 18; ++i) acc = acc + D[i] * mn[i];
-    const R acc1 = shup(acc, 1);
-    if (k == 2) acc = acc + acc1;
-    R lq = acc + (al * L + be * Lm + (shup(lds, 1) - lds));
-    if (!body) lq = R(0);
-    if (a.last) lq = lq + l0;                   // stage 1 read q = scp0
-    if (act && ti.own) {
-      if (!a.last) st_nt(a.lam0 + fo, cb + l, l0);
-      st_nt(a.lq + fo, cb + l, lq);
+  for (int i = 0; i < 19; ++i) row[i] = (((unsigned)I[R2_PLACEA + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch;
+  RingAdj<R> f;
+  ring_adj(m, I, K, a, c, l, f, [&](int i) { return lds_row<R>(smem_raw + sg.bytes + mb, row[i]); });
+  __syncthreads();
+  for (int n = ti.n0; n < ti.n1; ++n) {
+    const unsigned char *buf = smem_raw + ((n - ti.n0) & 1) * sg.bytes + lb;
+    const R mr = lds_row<R>(buf, row[18]);
+    const R p = pn, q2 = qn;
+    const bool more = n + 1 < ti.n1;
+    if (more) fetch(n + 1);
+    R mu, nucc;
+    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i) { return lds_row<R>(buf, row[i]); });
+    ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
+    if (more) {
+      st_.put(smem_raw + ((n + 1 - ti.n0) & 1) * sg.bytes);
+      __syncthreads();
     }
   }
 }

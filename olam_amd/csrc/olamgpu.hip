@@ -720,8 +720,11 @@ struct Impl : ImplBase {
   // offsets), meshes with other neighbourhoods than pentagons and hexagons, and when one
   // of them is asked for by name.
   bool use_ring2 = false;
-  DevBuf b_r2cell, b_r2kf, b_r2face, b_r2out, b_r2ka, b_vr;
+  DevBuf b_r2ints, b_r2kf, b_r2ka, b_vr;
   Ring2Tab<R> r2{};
+  bool r2_stagef = false, r2_stagea = false;     // rows staged in LDS, forward and adjoint
+  DevBuf b_r2n[2], b_r2cells[2];
+  Ring2Stage r2f{}, r2a{};
   // state
   DevBuf thil[2], wmc, wc, vxe, vye, vze, vmc, vc, vmasc, wmasc, alpha, pwfac, pvfac, thilt, vmxet, vmyet, vmzet, vmt;
   DevBuf rho, press, rho_old;
@@ -790,6 +793,10 @@ struct Impl : ImplBase {
   // L=60, 10 tracers: 1 -> 151, 2 -> 121, 5 -> 107, 10 -> 104 ms per step, because the
   // per-column gathers of winds and metrics are shared); OLAMGPU_TPW overrides
   int tpw = 16;
+  // the two-ring kernels: blocks of nwv waves by tracer groups
+  dim3 ring2_grid(int nwv) const {
+    return dim3((unsigned)(((long)nw * halves + nwv - 1) / nwv), (unsigned)((std::max(ntr, 1) + tpw - 1) / tpw));
+  }
   unsigned nblk_tr() const { int ng = (std::max(ntr, 1) + tpw - 1) / tpw; return nblk(nw * ng); }
 
   Impl(const olamgpu_mesh *m, const olamgpu_params *p, hipStream_t st, Prof *pr, Topo &&topo)
@@ -826,7 +833,7 @@ struct Impl : ImplBase {
     }
     if (use_patch) build_patch_tables();
     use_ring2 = prm.scal_horiz_adv_order >= 2 && ntr > 0 && !(use_patch || two_pass || fused_fwd || !fuse_adj) &&
-                mza <= RING2_TALL_MZA && wsz * sizeof(R) < (size_t(1) << 32);
+                mza <= RING2_TALL_MZA && std::max(wsz, vsz) * sizeof(R) < (size_t(1) << 32);
     if (use_ring2) build_ring2_tables(m);
   }
 
@@ -852,15 +859,31 @@ struct Impl : ImplBase {
       const int side = m->w_dirv[(size_t)(oc + 1) * 7 + i] < 0.f ? 0 : 1;
       for (int q = 0; q < nt; ++q) o[q] = offs[q][(size_t)(v + 1) * 2 + side];
     };
-    std::vector<R> kf((size_t)nw * 36, R(0)), ka((size_t)nw * 42, R(0));
+    const int nkf = r2_nkf(nt), KF = r2_kf(nt), COF = r2_cof(nt);
+    std::vector<R> kf((size_t)nw * nkf, R(0)), ka((size_t)nw * R2_NKA, R(0));
+    std::vector<int> ints((size_t)nw * R2_INTS, 0);
     parallel_ranges(nw, [&](int c0, int c1) {
       for (int c = c0; c < c1; ++c) {
         const int np = t.w_npoly[c];
+        int *I = &ints[(size_t)c * R2_INTS];
+        R *F = &kf[(size_t)c * nkf], *A = &ka[(size_t)c * R2_NKA];
+        std::copy_n(&t.w_nbr[(size_t)c * NSLOT], 6, I + R2_NBR);
+        std::copy_n(&h.cell[(size_t)c * 12], 12, I + R2_CELL);
+        std::copy_n(&t.w_face[(size_t)c * NSLOT], 6, I + R2_FACE);
+        std::copy_n(&h.face[(size_t)c * 24], 24, I + R2_OUTER);
+        I[R2_OUT] = (int)h.out[c];
+        I[R2_NPOLY] = np;
         double cs[5] = {};
         for (int j = 0; j < np; ++j) {
-          double x[5];
+          double x[5], o[5];
           cof(c, j, x);
-          for (int q = 0; q < nt; ++q) cs[q] += x[q];
+          off(c, j, o);
+          for (int q = 0; q < nt; ++q) {
+            cs[q] += x[q];
+            F[R2_OFF + 6 * q + j] = (R)o[q];
+            F[COF + 6 * q + j] = (R)x[q];
+          }
+          F[R2_DIRV + j] = A[R2_DIRV + j] = (R)m->w_dirv[(size_t)(t.perm_w[c] + 1) * 7 + j];
         }
         for (int j = 0; j < np; ++j) {
           const int n = t.w_nbr[(size_t)c * NSLOT + j];
@@ -871,7 +894,7 @@ struct Impl : ImplBase {
           off(c, j, oc);
           double own = 1.0;
           for (int q = 0; q < nt; ++q) own -= cs[q] * oc[q];
-          ka[(size_t)c * 42 + 36 + j] = (R)own;
+          A[R2_KOWN + j] = (R)own;
           for (int role = 0; role < RING2_ROLES; ++role) {
             if (sl[role] < 0) continue;
             double ci[5], oi[5], f = 0.0, a = 0.0;
@@ -879,17 +902,70 @@ struct Impl : ImplBase {
             off(n, sl[role], oi);
             for (int q = 0; q < nt; ++q) { f += ob[q] * ci[q]; a += cb[q] * oi[q]; }
             sum += f;
-            if (role > 0) kf[(size_t)c * 36 + j * 6 + role] = (R)f;
-            ka[(size_t)c * 42 + j * 6 + role] = (R)a;
+            if (role > 0) F[KF + j * 6 + role] = (R)f;
+            A[R2_KA + j * 6 + role] = (R)a;
           }
-          kf[(size_t)c * 36 + j * 6] = (R)sum;
+          F[KF + j * 6] = (R)sum;
         }
       }
     });
-    upv(b_r2cell, h.cell); upv(b_r2face, h.face); upv(b_r2out, h.out);
-    upv(b_r2kf, kf); upv(b_r2ka, ka);
-    r2.cell = dp<int>(b_r2cell); r2.face = dp<int>(b_r2face); r2.out = dp<unsigned>(b_r2out);
-    r2.kf = dp<R>(b_r2kf); r2.ka = dp<R>(b_r2ka);
+    // Staged rows pay from two tracers a wave and some 4,000 columns on.  Measured, staged
+    // against gathered, forward and adjoint stage in us (FP32, 60 levels, 256,002 columns):
+    // 1 tracer 218 / 216 and 326 / 288, 2 tracers 259 / 280 and 367 / 379, 10 tracers 662 /
+    // 926 and 890 / 1147; 10 tracers, 30 levels: 1,442 columns 15.1 / 14.1 and 15.5 / 14.9,
+    // 5,762 columns 21.9 / 26.7 and 22.0 / 29.7.
+    if (std::min(ntr, tpw) >= 2 && nw >= 4096) {
+      r2_stagef = build_ring2_stage(ints, RING2_NWF, R2_PLACE, b_r2n[0], b_r2cells[0], r2f);
+      r2_stagea = build_ring2_stage(ints, RING2_NWA, R2_PLACEA, b_r2n[1], b_r2cells[1], r2a);
+    }
+    upv(b_r2ints, ints); upv(b_r2kf, kf); upv(b_r2ka, ka);
+    r2.ints = dp<int>(b_r2ints); r2.kf = dp<R>(b_r2kf); r2.ka = dp<R>(b_r2ka);
+  }
+  // Row lists of the staged blocks of nwv waves: the columns of a block and of their
+  // rings, ascending, and at word `place` of each column's record the places of its cells
+  // in that list.  False where the rows of some block do not fit the kernel's registers or
+  // two buffers of them the LDS.
+  bool build_ring2_stage(std::vector<int> &ints, int nwv, int place, DevBuf &bn, DevBuf &bcells, Ring2Stage &sg) {
+    const int per = nwv / halves, nb = (nw + per - 1) / per;
+    std::vector<int> rows((size_t)nb * per * 19), cnt(nb, 0);
+    std::atomic<int> most{0};
+    parallel_ranges(nb, [&](int b0, int b1) {
+      for (int b = b0; b < b1; ++b) {
+        int *r = &rows[(size_t)b * per * 19], *e = r;
+        const int c1 = std::min(nw, (b + 1) * per);
+        for (int c = b * per; c < c1; ++c) {
+          *e++ = c;
+          e = std::copy_n(&ints[(size_t)c * R2_INTS], 18, e);
+        }
+        std::sort(r, e);
+        e = std::unique(r, e);
+        cnt[b] = (int)(e - r);
+        int have = most;
+        while (have < cnt[b] && !most.compare_exchange_weak(have, cnt[b])) {}
+        for (int c = b * per; c < c1; ++c) {
+          int *I = &ints[(size_t)c * R2_INTS];
+          for (int i = 0; i < 19; ++i) {
+            const unsigned at = (unsigned)(std::lower_bound(r, e, i < 18 ? I[i] : c) - r);
+            I[place + i / 4] |= (int)((at & 255u) << (8 * (i % 4)));
+          }
+        }
+      }
+    });
+    const int nmax = most;
+    const unsigned pitch = (unsigned)((mza * sizeof(R) + 15) / 16 * 16);
+    // a lane above the last row's levels still reads inside the buffer
+    const size_t data = (size_t)nmax * pitch, bytes = (data + (size_t)ldk * sizeof(R) + 1023) / 1024 * 1024;
+    int dev = 0, v = 0;
+    HIPCHK(hipGetDevice(&dev));
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0) v = 65536;
+    if (nmax > 256 || 2 * bytes > (size_t)v || data > (size_t)RING2_NCH * nwv * 1024) return false;
+    std::vector<int> cells((size_t)nb * nmax, 0);
+    for (int b = 0; b < nb; ++b) std::copy_n(&rows[(size_t)b * per * 19], cnt[b], &cells[(size_t)b * nmax]);
+    upv(bn, cnt); upv(bcells, cells);
+    sg.count = dp<int>(bn); sg.cells = dp<int>(bcells);
+    sg.nmax = nmax; sg.pitch = pitch; sg.magic = (unsigned)(((1ull << 32) + pitch - 1) / pitch);
+    sg.bytes = (unsigned)bytes;
+    return true;
   }
 
   // Patches of 8 * cpw columns (one block of 8 waves, cpw owned columns per wave),
@@ -1739,16 +1815,29 @@ struct Impl : ImplBase {
     have_fwd = true;
   }
 
+  // 16-byte pieces of the staged rows that a lane carries per tracer
+  static constexpr int RING2_NCH = sizeof(R) == 4 ? 2 : 4;
+  template <bool Q3, bool TALL> void ring2_fwd(const TrStage<R, RP> &a) {
+    if (r2_stagef)
+      LAUNCH_SH("k_tr_ring2s", (k_tr_ring2s<R, RP, Q3, TALL, RING2_NCH>), ring2_grid(RING2_NWF),
+                dim3(RING2_NWF * WAVE), 2 * r2f.bytes, dm, r2, r2f, a);
+    else LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, Q3, TALL>), ring2_grid(WPB), dim3(256), dm, r2, a);
+  }
+  template <bool TALL> void ring2_adj(const TrAdj<R, RP> &a, const AdjHist<R> &h) {
+    const R *vr = dp<R>(b_vr);
+    if (r2_stagea)
+      LAUNCH_SH("k_tr_ring2s_adj", (k_tr_ring2s_adj<R, RP, TALL, RING2_NCH>), ring2_grid(RING2_NWA),
+                dim3(RING2_NWA * WAVE), 2 * r2a.bytes, dm, r2, r2a, a, h, vr);
+    else LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, TALL>), ring2_grid(WPB), dim3(256), dm, r2, a, h, vr);
+  }
+
   // reconstruction coefficients of the stage input, then the update of the unlimited
   // tracers (grad_t2d or grad_t2d_quadratic, scalar_v_column + scalar_w_column)
   void tracer_update(const TrStage<R, RP> &a) {
     // a limited final stage keeps the gradients: the limiter passes read them
     if (use_ring2 && !a.lim) {
-      const bool q3 = a.order == 3;
-      if (q3 && dm.tall) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, true, true>), dim3(nblk_tr()), dim3(256), dm, r2, a);
-      else if (q3) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, true, false>), dim3(nblk_tr()), dim3(256), dm, r2, a);
-      else if (dm.tall) LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, false, true>), dim3(nblk_tr()), dim3(256), dm, r2, a);
-      else LAUNCH("k_tr_ring2", (k_tr_ring2<R, RP, false, false>), dim3(nblk_tr()), dim3(256), dm, r2, a);
+      if (dm.tall) a.order == 3 ? ring2_fwd<true, true>(a) : ring2_fwd<false, true>(a);
+      else a.order == 3 ? ring2_fwd<true, false>(a) : ring2_fwd<false, false>(a);
       return;
     }
     if (a.order < 3 && fused_fwd && !a.lim) {
@@ -1802,13 +1891,24 @@ struct Impl : ImplBase {
     RP *rho_tr = tracer_rho();
     if (use_ring2)
       LAUNCH("k_tr_vr", (k_tr_vr<R, RP>), dim3((unsigned)((wsz + 255) / 256)), dim3(256), dm, rho_tr, dp<R>(b_vr));
+    // Two-ring stages without implicit columns keep mu of every stage: they go from the
+    // current buffer X to the other (Y) and, in RK3, to lam0's (Z), and the last stage, which
+    // gathers from Y or Z and reads only its own columns of X and Y, writes X.  (The lanes of
+    // a tall column's wave that overlap the other wave may read what that one has written;
+    // they store nothing and no other lane uses their value.)
+    AdjHist<R> hist{};
+    hist.on = use_ring2 && !any_imp && !any_lim;
+    const DevBuf &hx = cur_adj_buf(), &hy = cur_adj ? adjA : adjB;
+    hist.mu3 = dp<R>(cur_adj_buf());
+    hist.dt3 = dtlr[nrk - 1];
+    if (nrk == 3) { hist.mu2 = hy.as<R>(); hist.dt2 = dtlr[1]; }
     // lam0 is not cleared: the first adjoint stage (a.first) starts it from zero
     for (int istage = nrk; istage >= 1; --istage) {
       TrAdj<R, RP> a;
-      DevBuf &muB = cur_adj_buf();
-      DevBuf &lqB = cur_adj ? adjA : adjB;
-      a.mu = dp<R>(muB); a.lam0 = dp<R>(lam0); a.nu = dp<R>(nu); a.lpart = dp<R>(lpart);
-      a.lgx = dp<R>(lgG); a.lgy = dp<R>(lgG) + (size_t)std::max(ntr, 1) * tstride; a.lq = dp<R>(lqB);
+      const DevBuf &muB = !hist.on ? cur_adj_buf() : (istage == nrk ? hx : (istage == nrk - 1 ? hy : lam0));
+      const DevBuf &lqB = !hist.on ? (cur_adj ? adjA : adjB) : (istage == 1 ? hx : (istage == nrk ? hy : lam0));
+      a.mu = muB.as<R>(); a.lam0 = dp<R>(lam0); a.nu = dp<R>(nu); a.lpart = dp<R>(lpart);
+      a.lgx = dp<R>(lgG); a.lgy = dp<R>(lgG) + (size_t)std::max(ntr, 1) * tstride; a.lq = lqB.as<R>();
       for (int t = 0; t < 3; ++t) a.lgq[t] = dp<R>(lgq[t]);
       a.vmasc = dp<R>(vmasc); a.wmasc = dp<R>(wmasc); a.rho_old = dp<R>(rho_old); a.ffimp = dp<R>(ffimp);
       a.rho = rho_tr;
@@ -1834,17 +1934,13 @@ struct Impl : ImplBase {
         else if (pa.cpw == 2) LAUNCH_SH("k_tr_adj_patch", (k_tr_adj_patch<R, RP, 2>), g, b, pa.lds, dm, a, pa.tab);
         else LAUNCH_SH("k_tr_adj_patch", (k_tr_adj_patch<R, RP, 1>), g, b, pa.lds, dm, a, pa.tab);
       } else if (use_ring2) {
-        const bool q3 = a.order == 3;
-        const R *vr = dp<R>(b_vr);
-        if (q3 && dm.tall) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, true, true>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
-        else if (q3) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, true, false>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
-        else if (dm.tall) LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, false, true>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
-        else LAUNCH("k_tr_ring2_adj", (k_tr_ring2_adj<R, RP, false, false>), dim3(nblk_tr()), dim3(256), dm, r2, a, vr);
+        if (dm.tall) ring2_adj<true>(a, hist);
+        else ring2_adj<false>(a, hist);
       } else {
         adjoint_faces(a);
         adjoint_coefs(a);
       }
-      cur_adj = 1 - cur_adj;
+      if (!hist.on) cur_adj = 1 - cur_adj;
     }
     // the diffusion tendency was built from the tracers before the step
     if (sgs)
