@@ -20,6 +20,7 @@
 #include <string>
 #include <system_error>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/olamgpu.h"
@@ -2066,16 +2067,28 @@ __global__ void k_scale(R *a, long n, R f, int mza, int ldk, int klo, int khi) {
   int k = (int)(i % ldk) + 1;
   if (k >= klo && k <= khi) a[i] = a[i] / f;
 }
-// dense (n, mza) original order <-> device (n, ldk) renumbered
-template <class T>
-__global__ void k_perm_copy(const int *inv, T *dev, T *dense, int n, int mza, int ldk, int dir) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)n * mza) return;
-  long o = i / mza;
-  int l = (int)(i % mza);
-  long d = (long)inv[o] * ldk + l;
-  if (dir == 0) dense[i] = dev[d];
-  else dev[d] = dense[i];
+// dense (n, mza) original order <-> device (n, ldk) renumbered.  A wave moves PERM_N
+// points, one row of levels after another with every load issued before the first store.
+// Measured at 400,002 columns and 60 levels (W field 0.20 GB moved, V field 0.60), out /
+// in: 0.045 / 0.033 and 0.207 / 0.157 ms, against 0.055 / 0.054 and 0.244 / 0.246 with one
+// element a thread and a 64-bit division each.
+constexpr int PERM_N = 2;
+template <class T, int DIR>
+__global__ __launch_bounds__(256) void k_perm_copy(const int *inv, T *dev, T *dense, int n, int mza, int ldk) {
+  const int o0 = (blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * PERM_N;
+  const int cnt = min(PERM_N, n - o0);
+  for (int l = lane_id(); l < mza; l += WAVE) {
+    T v[PERM_N];
+#pragma unroll
+    for (int i = 0; i < PERM_N; ++i)
+      if (i < cnt) v[i] = DIR ? dense[(long)(o0 + i) * mza + l] : dev[(long)inv[o0 + i] * ldk + l];
+#pragma unroll
+    for (int i = 0; i < PERM_N; ++i)
+      if (i < cnt) {
+        if constexpr (DIR) dev[(long)inv[o0 + i] * ldk + l] = v[i];
+        else dense[(long)(o0 + i) * mza + l] = v[i];
+      }
+  }
 }
 
 template <class R, class RP>
@@ -2119,15 +2132,15 @@ void Impl<R, RP>::copy_field(int id, int index, void *buf, int dir, int *eb) {
   }
   int n = isv ? nv : nw;
   const int *dinv = isv ? b_invv.as<int>() : b_invw.as<int>();
-  long tot = (long)n * mza;
-  unsigned g = (unsigned)((tot + 255) / 256);
-  if (isrp) {
-    if (eb) *eb = sizeof(RP);
-    LAUNCH("k_perm_copy", k_perm_copy<RP>, dim3(g), dim3(256), dinv, b->as<RP>() + off, (RP *)buf, n, mza, ldk, dir);
-  } else {
-    if (eb) *eb = sizeof(R);
-    LAUNCH("k_perm_copy", k_perm_copy<R>, dim3(g), dim3(256), dinv, b->as<R>() + off, (R *)buf, n, mza, ldk, dir);
-  }
+  const unsigned g = (unsigned)((n + WPB * PERM_N - 1) / (WPB * PERM_N));
+  auto move = [&](auto *dev) {
+    using T = std::remove_pointer_t<decltype(dev)>;
+    if (eb) *eb = sizeof(T);
+    if (dir) LAUNCH("k_perm_copy", (k_perm_copy<T, 1>), dim3(g), dim3(256), dinv, dev, (T *)buf, n, mza, ldk);
+    else LAUNCH("k_perm_copy", (k_perm_copy<T, 0>), dim3(g), dim3(256), dinv, dev, (T *)buf, n, mza, ldk);
+  };
+  if (isrp) move(b->as<RP>() + off);
+  else move(b->as<R>() + off);
   HIPCHK(hipGetLastError());
 }
 
