@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -66,6 +67,7 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { if (p) (void)hipFree(p); }
   void alloc(size_t b) {
+    if (p && bytes == b) return;                          // a new upload of the same size
     if (p) { (void)hipFree(p); p = nullptr; }
     bytes = b;
     if (b) HIPCHK(hipMalloc(&p, b));
@@ -75,10 +77,14 @@ struct DevBuf {
 
 // ------------------------------------------------------------------ host transfers
 // A host array in the reference's Fortran layout (mza, n + 1), dummy column first, moves
-// as raw bytes between host memory and a device staging buffer through two pinned
-// bounce buffers (the host-side copy of one chunk overlaps the DMA of the other, and
-// the host-side copy is split over threads); kernels then convert it to or from the
-// device layout, renumbered columns of ldk levels (levels mza..ldk-1 zero).
+// as raw bytes between host memory and a device staging buffer through a ring of pinned
+// bounce buffers; kernels convert it to or from the device layout, renumbered columns of
+// ldk levels (levels mza..ldk-1 zero).  The host-side copy of one chunk, split over a
+// context's copy threads, overlaps the DMA of the others, across the arrays of a call.
+// What bounds it is the host copy and the PCIe link, one after the other only at a call's
+// ends.  A host's long step on 40,962 columns, 60 levels and 10 tracers (0.17 GB up, 0.19
+// down) takes 14.1 ms, 18.2 with two 64 MiB buffers, a wait per array and threads spawned
+// per chunk.
 template <class D, class H>
 __global__ __launch_bounds__(256) void k_unpack(D *dst, const H *src, const int *perm, int n, int mza, int ldk) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -94,73 +100,140 @@ __global__ __launch_bounds__(256) void k_pack(H *dst, const D *src, const int *i
   dst[i] = j == 0 ? H(0) : (H)src[(size_t)inv[j - 1] * ldk + l];
 }
 
+// Threads that share one host copy with the caller.  They belong to one context, start with
+// its first large transfer, wait between copies (a short spin, so that the chunks of one
+// transfer find them awake, then asleep) and end with the context.  Spawning them for each
+// chunk cost as much as a 10 MB copy.
+struct CopyPool {
+  static constexpr size_t PART = size_t(256) << 10;      // least bytes worth a thread
+  std::vector<std::thread> th;
+  std::mutex mu;
+  std::condition_variable cv;
+  std::atomic<unsigned> gen{0};
+  std::atomic<int> left{0};
+  std::atomic<bool> stop{false};
+  char *dst = nullptr;
+  const char *src = nullptr;
+  size_t part = 0, total = 0;
+  int parts = 1;
+  ~CopyPool() {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      stop = true;
+    }
+    cv.notify_all();
+    for (auto &t : th) t.join();
+  }
+  void slice(int k) const {
+    const size_t o = (size_t)k * part;
+    if (o < total) std::memcpy(dst + o, src + o, std::min(part, total - o));
+  }
+  void run(int k) {
+    unsigned seen = 0;
+    for (;;) {
+      for (int i = 0; i < 20000 && gen.load(std::memory_order_acquire) == seen && !stop; ++i) __builtin_ia32_pause();
+      if (gen.load(std::memory_order_acquire) == seen) {
+        std::unique_lock<std::mutex> lock(mu);
+        cv.wait(lock, [&] { return gen.load(std::memory_order_acquire) != seen || stop; });
+      }
+      if (stop) return;
+      seen = gen.load(std::memory_order_acquire);
+      if (k < parts) slice(k);
+      left.fetch_sub(1, std::memory_order_release);
+    }
+  }
+  void start() {
+    const int n = (int)std::max(1u, std::min(8u, std::thread::hardware_concurrency())) - 1;
+    th.reserve(n);
+    try {
+      while ((int)th.size() < n) th.emplace_back(&CopyPool::run, this, (int)th.size() + 1);
+    } catch (const std::system_error &) {                 // fewer threads than wished
+    }
+  }
+  // one caller at a time (the context's)
+  void copy(void *d, const void *s, size_t nb) {
+    const int want = (int)std::min<size_t>(th.size() + 1, nb / PART);
+    if (want < 2) { std::memcpy(d, s, nb); return; }
+    dst = (char *)d; src = (const char *)s; total = nb; parts = want;
+    part = ((nb + want - 1) / want + 63) / 64 * 64;
+    left.store((int)th.size(), std::memory_order_relaxed);
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      gen.fetch_add(1, std::memory_order_release);
+    }
+    cv.notify_all();
+    slice(0);
+    while (left.load(std::memory_order_acquire) > 0) __builtin_ia32_pause();
+  }
+};
+
 struct HostXfer {
-  static constexpr size_t CHUNK = size_t(64) << 20;
-  void *pin[2] = {nullptr, nullptr};
-  hipEvent_t ev[2] = {nullptr, nullptr};
+  // 4 MiB: a chunk's DMA (80 us) and its copy by 8 threads are of one length
+  static constexpr size_t CHUNK = size_t(4) << 20;
+  static constexpr int RING = 4;
+  void *pin[RING] = {};
+  hipEvent_t ev[RING] = {};
+  struct { void *dst; size_t nb; } out[RING] = {};        // device-to-host chunks under way
+  unsigned next = 0;
   DevBuf stage;
-  int nthr = 1;
+  CopyPool pool;
   ~HostXfer() {
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < RING; ++k) {
       if (pin[k]) (void)hipHostFree(pin[k]);
       if (ev[k]) (void)hipEventDestroy(ev[k]);
     }
   }
   void ready(size_t bytes, hipStream_t s) {
-    if (!pin[0]) {
-      for (int k = 0; k < 2; ++k) {
-        HIPCHK(hipHostMalloc(&pin[k], CHUNK, hipHostMallocDefault));
-        HIPCHK(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
+    if (!ev[RING - 1]) {
+      for (int k = 0; k < RING; ++k) {
+        if (!pin[k]) HIPCHK(hipHostMalloc(&pin[k], CHUNK, hipHostMallocDefault));
+        if (!ev[k]) HIPCHK(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
         HIPCHK(hipEventRecord(ev[k], s));
       }
-      nthr = (int)std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+      pool.start();
     }
-    if (stage.bytes < bytes) stage.alloc(bytes);
-  }
-  void copy(void *dst, const void *src, size_t nb) const {
-    const size_t part = (nb + nthr - 1) / nthr;
-    if (nthr == 1 || nb < (size_t(4) << 20)) { std::memcpy(dst, src, nb); return; }
-    std::vector<std::thread> th;
-    for (int k = 0; k < nthr; ++k) {
-      const size_t o = (size_t)k * part;
-      if (o >= nb) break;
-      th.emplace_back([=] { std::memcpy((char *)dst + o, (const char *)src + o, std::min(part, nb - o)); });
+    // a larger staging buffer: what the stream still does with the old one comes first
+    if (stage.bytes < bytes) {
+      HIPCHK(hipStreamSynchronize(s));
+      stage.alloc(bytes);
     }
-    for (auto &x : th) x.join();
   }
-  // host -> stage
+  // the next ring slot, its earlier DMA ended and its data delivered
+  int slot() {
+    const int k = (int)(next++ % RING);
+    HIPCHK(hipEventSynchronize(ev[k]));
+    if (out[k].dst) { pool.copy(out[k].dst, pin[k], out[k].nb); out[k].dst = nullptr; }
+    return k;
+  }
+  // host -> stage: h may be reused on return
   void up(const void *h, size_t bytes, hipStream_t s) {
     ready(bytes, s);
-    for (size_t o = 0, i = 0; o < bytes; o += CHUNK, ++i) {
-      const int k = (int)(i & 1);
+    for (size_t o = 0; o < bytes; o += CHUNK) {
+      const int k = slot();
       const size_t nb = std::min(CHUNK, bytes - o);
-      HIPCHK(hipEventSynchronize(ev[k]));          // the DMA that last read pin[k] is done
-      copy(pin[k], (const char *)h + o, nb);
+      pool.copy(pin[k], (const char *)h + o, nb);
       HIPCHK(hipMemcpyAsync((char *)stage.p + o, pin[k], nb, hipMemcpyHostToDevice, s));
       HIPCHK(hipEventRecord(ev[k], s));
     }
   }
-  // stage -> host (the stream's earlier work, the packing kernel, comes first)
+  // stage -> host (the stream's earlier work, the packing kernel, comes first); the last
+  // chunks arrive with finish()
   void down(void *h, size_t bytes, hipStream_t s) {
-    ready(bytes, s);
-    size_t prev_o = 0, prev_nb = 0;
-    int prev_k = -1;
-    for (size_t o = 0, i = 0; o < bytes; o += CHUNK, ++i) {
-      const int k = (int)(i & 1);
+    for (size_t o = 0; o < bytes; o += CHUNK) {
+      const int k = slot();
       const size_t nb = std::min(CHUNK, bytes - o);
       HIPCHK(hipMemcpyAsync(pin[k], (const char *)stage.p + o, nb, hipMemcpyDeviceToHost, s));
       HIPCHK(hipEventRecord(ev[k], s));
-      if (prev_k >= 0) {
-        HIPCHK(hipEventSynchronize(ev[prev_k]));
-        copy((char *)h + prev_o, pin[prev_k], prev_nb);
-      }
-      prev_k = k; prev_o = o; prev_nb = nb;
-    }
-    if (prev_k >= 0) {
-      HIPCHK(hipEventSynchronize(ev[prev_k]));
-      copy((char *)h + prev_o, pin[prev_k], prev_nb);
+      out[k].dst = (char *)h + o;
+      out[k].nb = nb;
     }
   }
+  void finish() {
+    if (!ev[RING - 1]) return;
+    for (int i = 0; i < RING; ++i) (void)slot();
+  }
+  // after an error: nothing may be delivered to host arrays later
+  void drop() { for (auto &o : out) o.dst = nullptr; }
 };
 
 // ------------------------------------------------------------------ kernel timing
@@ -611,6 +684,7 @@ struct ImplBase {
   virtual void set_sgsmix(int, int) = 0;
   virtual void tracer_maxmin(float *) = 0;
   virtual void mass_sums_noalloc(double *, double *) = 0;
+  virtual void drop_transfers() = 0;
 };
 
 // x**n for an integer n >= 0 in the type of x, one rounding per factor (Fortran's
@@ -1114,32 +1188,34 @@ struct Impl : ImplBase {
       lev8[0][l] = m->zwgt_top8[l]; lev8[1][l] = m->zwgt_bot8[l];
       lev8[2][l] = m->gdz_wgtm8[l]; lev8[3][l] = m->gdz_wgtp8[l];
     }
-    // control volumes
-    std::vector<R> arw(wsz, 0), volti(wsz, 0), volwi(wsz, 0), arv(vsz, 0), volvi(vsz, 0);
-    std::vector<double> volt(wsz, 0);
-    for (int c = 0; c < nw; ++c) {
-      size_t fo = (size_t)(t.perm_w[c] + 1) * mza;
-      for (int l = 0; l < mza; ++l) {
-        size_t i = (size_t)c * ldk + l;
-        arw[i] = m->arw[fo + l];
-        volt[i] = m->volt[fo + l];
-        if (!f64) { volti[i] = m->volti[fo + l]; volwi[i] = m->volwi[fo + l]; }
-      }
-      if (f64) {   // inverse volumes rebuilt from volt in double (see olamgpu.h)
-        for (int k = 2; k <= mza; ++k) volti[(size_t)c * ldk + k - 1] = (R)(1.0 / volt[(size_t)c * ldk + k - 1]);
-        for (int k = 2; k <= mza - 1; ++k)
-          volwi[(size_t)c * ldk + k - 1] = (R)(1.0 / (volt[(size_t)c * ldk + k - 1] + volt[(size_t)c * ldk + k]));
-      }
-    }
-    for (int e = 0; e < nv; ++e) {
-      size_t fo = (size_t)(t.perm_v[e] + 1) * mza;
-      int w1 = t.v_iw[e * 2], w2 = t.v_iw[e * 2 + 1];
-      for (int l = 0; l < mza; ++l) {
-        size_t i = (size_t)e * ldk + l;
-        arv[i] = m->arv[fo + l];
-        if (!f64) volvi[i] = m->volvi[fo + l];
-        else if (l >= 1) volvi[i] = (R)(1.0 / (volt[(size_t)w1 * ldk + l] + volt[(size_t)w2 * ldk + l]));
-      }
+    // control volumes, repacked on the device; the FP64 mode's inverse volumes here
+    b_arw.alloc(wsz * sizeof(R)); b_volti.alloc(wsz * sizeof(R)); b_volwi.alloc(wsz * sizeof(R));
+    b_volt.alloc(wsz * sizeof(double)); b_arv.alloc(vsz * sizeof(R)); b_volvi.alloc(vsz * sizeof(R));
+    h2d<R>(b_arw, m->arw, t.perm_w);
+    h2d<double>(b_volt, m->volt, t.perm_w);
+    h2d<R>(b_arv, m->arv, t.perm_v);
+    if (!f64) {
+      h2d<R>(b_volti, m->volti, t.perm_w);
+      h2d<R>(b_volwi, m->volwi, t.perm_w);
+      h2d<R>(b_volvi, m->volvi, t.perm_v);
+    } else {   // inverse volumes rebuilt from volt in double (see olamgpu.h)
+      std::vector<R> volti(wsz, 0), volwi(wsz, 0), volvi(vsz, 0);
+      auto vol = [&](int c) { return m->volt + (size_t)(t.perm_w[c] + 1) * mza; };
+      parallel_ranges(nw, [&](int c0, int c1) {
+        for (int c = c0; c < c1; ++c) {
+          const double *v = vol(c);
+          R *o = &volti[(size_t)c * ldk], *ow = &volwi[(size_t)c * ldk];
+          for (int k = 2; k <= mza; ++k) o[k - 1] = (R)(1.0 / v[k - 1]);
+          for (int k = 2; k <= mza - 1; ++k) ow[k - 1] = (R)(1.0 / (v[k - 1] + v[k]));
+        }
+      });
+      parallel_ranges(nv, [&](int e0, int e1) {
+        for (int e = e0; e < e1; ++e) {
+          const double *v1 = vol(t.v_iw[e * 2]), *v2 = vol(t.v_iw[e * 2 + 1]);
+          for (int l = 1; l < mza; ++l) volvi[(size_t)e * ldk + l] = (R)(1.0 / (v1[l] + v2[l]));
+        }
+      });
+      upv(b_volti, volti); upv(b_volwi, volwi); upv(b_volvi, volvi);
     }
     upv(b_npoly, t.w_npoly); upv(b_nbr, t.w_nbr); upv(b_face, t.w_face); upv(b_back, t.w_back);
     upv(b_viw, t.v_iw); upv(b_vim, t.v_im); upv(b_miv, t.m_iv); upv(b_mim, t.m_im); upv(b_invw, t.inv_w); upv(b_invv, t.inv_v);
@@ -1162,7 +1238,6 @@ struct Impl : ImplBase {
     upv(b_vfact, vfact); upv(b_xxyym, xxyym);
     for (int i = 0; i < 11; ++i) upv(b_lev[i], lev[i]);
     for (int i = 0; i < 4; ++i) upv(b_lev8[i], lev8[i]);
-    upv(b_arw, arw); upv(b_volti, volti); upv(b_volwi, volwi); upv(b_volt, volt); upv(b_arv, arv); upv(b_volvi, volvi);
     for (int b = 0; b < 2; ++b) {
       for (int q = 0; q < 5; ++q) upv(b_q[b][q], q3[b][q]);
       for (int q = 0; q < 3; ++q) { upv(b_os[b][q], os3[b][q]); upv(b_on[b][q], on3[b][q]); }
@@ -1234,7 +1309,8 @@ struct Impl : ImplBase {
       R factr = R(0);
       if (rf.dorayfdiv && do_div) factr = (R)(std::max(prm.divh_damp_fact, prm.rayfdiv_fact) / (R)dtm);
       else if (rf.dorayfdiv) factr = (R)(prm.rayfdiv_fact / (R)dtm);
-      for (int e = 0; e < nv; ++e) {
+      parallel_ranges(nv, [&](int e0, int e1) {
+      for (int e = e0; e < e1; ++e) {
         int o = t.perm_v[e] + 1;
         int w1o = in.viw(0, o - 1) + 1, w2o = in.viw(1, o - 1) + 1;
         const double factb = do_divh ? facth * (double)ipow((R)std::min(m->arw0[w1o], m->arw0[w2o]), dl - 1) : 0.0;
@@ -1249,6 +1325,7 @@ struct Impl : ImplBase {
                                               (double)(R(1) - zf));
         }
       }
+      });
       if (do_divl) upv(fdivl, fl);
       if (do_divh) upv(fdivh, fh);
       // the divergence and its Laplacians; a third buffer keeps the divergence for
@@ -1356,7 +1433,6 @@ struct Impl : ImplBase {
     hipLaunchKernelGGL((k_unpack<D, H>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s,
                        (D *)dst, xfer.stage.as<const H>(), dev_perm(perm, false), n, mza, ldk);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s));
   }
   template <class D, class H> void h2d(DevBuf &b, const H *h, const std::vector<int> &perm) {
     h2d_at<D>(b.p, h, perm);
@@ -1364,6 +1440,7 @@ struct Impl : ImplBase {
   template <class D, class H> void h2d_off(DevBuf &b, size_t off, const H *h, const std::vector<int> &perm) {
     h2d_at<D>((char *)b.p + off * sizeof(D), h, perm);
   }
+  // (callers end with xfer.finish())
   template <class D, class H> void d2h(const DevBuf &b, H *h, const std::vector<int> &perm, size_t off = 0) {
     const int n = (int)perm.size();
     const size_t cnt = (size_t)(n + 1) * mza;
@@ -1397,6 +1474,7 @@ struct Impl : ImplBase {
     V(vmc, h->vmc); V(vc, h->vc); W(wmasc, h->wmasc); V(vmasc, h->vmasc);
     W(alpha, h->alpha_press); W(pwfac, h->pwfac); V(pvfac, h->pvfac);
     W(thilt, h->thilt); W(vmxet, h->vmxet); W(vmyet, h->vmyet); W(vmzet, h->vmzet); V(vmt, h->vmt);
+    xfer.finish();
   }
   void check_n(int n) { if (n < 1 || n > ntr) throw Err(OLAMGPU_EINVAL, "scalar index out of range"); }
   void upload_scalar(int n, const float *p, const float *tt) override {
@@ -1410,7 +1488,11 @@ struct Impl : ImplBase {
       HIPCHK(hipMemsetAsync((char *)trsct.p + (size_t)(n - 1) * tstride * sizeof(R), 0, wsz * sizeof(R), s));
     }
   }
-  void download_scalar(int n, float *p) override { check_n(n); d2h<R>(trS, p, t.perm_w, (size_t)(n - 1) * tstride); }
+  void download_scalar(int n, float *p) override {
+    check_n(n);
+    d2h<R>(trS, p, t.perm_w, (size_t)(n - 1) * tstride);
+    xfer.finish();
+  }
   DevBuf &cur_adj_buf() { return cur_adj ? adjB : adjA; }
   void upload_adj(int n, const float *p) override {
     check_n(n); alloc_adj();
@@ -1419,6 +1501,7 @@ struct Impl : ImplBase {
   void download_adj(int n, float *p) override {
     check_n(n); alloc_adj();
     d2h<R>(cur_adj_buf(), p, t.perm_w, (size_t)(n - 1) * tstride);
+    xfer.finish();
   }
 
   // -------------------------------------------------------------- tend0 etc.
@@ -2007,6 +2090,7 @@ struct Impl : ImplBase {
   }
 
   void copy_field(int id, int index, void *buf, int dir, int *eb) override;
+  void drop_transfers() override { xfer.drop(); }
 
   // -------------------------------------------------------------- checkpoints
   // STATE: every field that the library's own calls modify and read back later
@@ -2174,9 +2258,11 @@ static int guarded(olamgpu_ctx *c, F &&f) {
     c->prof.flush();
     return OLAMGPU_OK;
   } catch (const Err &e) {
+    if (c->impl) c->impl->drop_transfers();
     c->err = e.what();
     return e.code;
   } catch (const std::exception &e) {
+    if (c->impl) c->impl->drop_transfers();
     c->err = e.what();
     return OLAMGPU_EHIP;
   }
