@@ -15,6 +15,7 @@
 // high-order correction vanishes the scale is arbitrary for the forward step but not
 // for the frozen adjoint, so the scales must come out exactly as in the oracle.
 #pragma once
+#include <type_traits>
 #include "kernels_tracer.h"
 
 template <class R>
@@ -99,9 +100,56 @@ __device__ __forceinline__ void lim_face(const DMesh<R> &m, const TrStage<R, RP>
   sf = vm * hiv;
 }
 
-template <class R, class RP>
+// What the faces of a column read of its neighbours at orders 1 and 2, loaded for every
+// face before the first is formed: with the loads under the upwind test (lim_face, kept for
+// order 3, whose nine more terms a face would not fit the registers) each face waited for
+// its own: 0.54 ms in k_tr_lim_scales and 0.77 in k_tr_lim_update at 40,962 columns, 41
+// levels and 5 tracers, 0.21 and 0.39 now.
+template <class R>
+struct LimNbr {
+  R q[7], q0[7], gx[7], gy[7];
+};
+template <int J0, int J1, class R, class RP>
+__device__ __forceinline__ void lim_nbr(const DMesh<R> &m, const TrStage<R, RP> &a, const LimCol<R> &L, long off,
+                                        int l, LimNbr<R> &N) {
+#pragma unroll
+  for (int j = J0; j < J1; ++j) {
+    N.q[j] = N.q0[j] = N.gx[j] = N.gy[j] = R(0);
+    if (j < 6 || L.np > 6) {
+      const long nb = off + (long)L.nb[j] * m.ldk;
+      N.q0[j] = ldl(a.q0 + nb, (unsigned)l);
+      N.q[j] = ldl(a.q_in + nb, (unsigned)l);
+      if (a.order > 1) {
+        N.gx[j] = ldl(a.gx + nb, (unsigned)l);
+        N.gy[j] = ldl(a.gy + nb, (unsigned)l);
+      }
+    }
+  }
+}
+// lim_face from loaded neighbours (the same expressions)
+template <class R>
+__device__ __forceinline__ void lim_face12(const LimCol<R> &L, const LimNbr<R> &N, int j, int order, int mode, R qc,
+                                           R q0c, R gxc, R gyc, R &low, R &hiv, R &sf, R &q0n) {
+  NOCONTRACT
+  const R vm = L.vm[j];
+  const bool iw1side = L.dv[j] < R(0);
+  const bool up_c = iw1side ? !(vm < R(0)) : (vm < R(0));
+  q0n = N.q0[j];
+  low = up_c ? q0c : q0n;
+  const bool hi_c = (mode == 2 && order == 1) ? iw1side : up_c;
+  R hs = qc, hn = N.q[j];
+  if (order > 1) {
+    hs = qc + L.dxs[j] * gxc + L.dys[j] * gyc;
+    hn = N.q[j] + L.dxn[j] * N.gx[j] + L.dyn[j] * N.gy[j];
+  }
+  hiv = (hi_c ? hs : hn) - low;
+  sf = vm * hiv;
+}
+
+template <class R, class RP, bool Q3, bool TALL>
 __global__ __launch_bounds__(256) void k_tr_lim_scales(DMesh<R> m, TrStage<R, RP> a, TrLim<R> T) {
   NOCONTRACT
+  m.tall = TALL;          // known to the compiler: one-wave columns carry no exchange code
   const TrItem ti = tr_item(m.nw, a.ntr, a.tpw, m.tall);
   const int c = ti.c;
   if (c >= m.nw) return;
@@ -120,8 +168,12 @@ __global__ __launch_bounds__(256) void k_tr_lim_scales(DMesh<R> m, TrStage<R, RP
     const R qc = ld(a.q_in + off, ic, act), q0c = ld(a.q0 + off, ic, act);
     R gxc = R(0), gyc = R(0), gqc[3] = {R(0), R(0), R(0)};
     if (a.order > 1) { gxc = ld(a.gx + off, ic, act); gyc = ld(a.gy + off, ic, act); }
-    if (a.order == 3)
+    LimNbr<R> N;
+    if constexpr (Q3) {
       for (int t = 0; t < 3; ++t) gqc[t] = ld(a.gq[t] + off, ic, act);
+    } else {
+      lim_nbr<0, 7>(m, a, L, off, l, N);
+    }
     // vertical: low-order upwind values from scp0, high-order from the stage input
     const R q0p1 = vshdn(m.tall, q0c, 1), qp1 = vshdn(m.tall, qc, 1);
     R upwl = (L.wm < R(0)) ? q0p1 : q0c;
@@ -143,7 +195,8 @@ __global__ __launch_bounds__(256) void k_tr_lim_scales(DMesh<R> m, TrStage<R, RP
     R fl = R(0), fin = R(0), fout = R(0);
     for_slots(L.np, [&](int j) {
       R low, hiv, sf, q0n;
-      lim_face(m, a, L, j, off, l, act, mode, qc, q0c, gxc, gyc, gqc, low, hiv, sf, q0n);
+      if constexpr (Q3) lim_face(m, a, L, j, off, l, act, mode, qc, q0c, gxc, gyc, gqc, low, hiv, sf, q0n);
+      else lim_face12(L, N, j, a.order, mode, qc, q0c, gxc, gyc, low, hiv, sf, q0n);
       const R d = L.dv[j];
       fl = fl + d * L.vm[j] * (low - q0c);
       if (mode == 1) fin = fin + fmax(d * sf, R(0));
@@ -193,9 +246,10 @@ __global__ __launch_bounds__(256) void k_tr_lim_scales(DMesh<R> m, TrStage<R, RP
   }
 }
 
-template <class R, class RP>
+template <class R, class RP, bool Q3, bool TALL>
 __global__ __launch_bounds__(256) void k_tr_lim_update(DMesh<R> m, TrStage<R, RP> a, TrLim<R> T) {
   NOCONTRACT
+  m.tall = TALL;          // known to the compiler: one-wave columns carry no exchange code
   const TrItem ti = tr_item(m.nw, a.ntr, a.tpw, m.tall);
   const int c = ti.c;
   if (c >= m.nw) return;
@@ -212,19 +266,37 @@ __global__ __launch_bounds__(256) void k_tr_lim_update(DMesh<R> m, TrStage<R, RP
     const R qc = ld(a.q_in + off, ic, act), q0c = ld(a.q0 + off, ic, act);
     R gxc = R(0), gyc = R(0), gqc[3] = {R(0), R(0), R(0)};
     if (a.order > 1) { gxc = ld(a.gx + off, ic, act); gyc = ld(a.gy + off, ic, act); }
-    if (a.order == 3)
+    LimNbr<R> N;
+    if constexpr (Q3)
       for (int t = 0; t < 3; ++t) gqc[t] = ld(a.gq[t] + off, ic, act);
     const R s1c = ldv(T.s1, off + ic, body, R(1));
     const R s2c = (mode == 1) ? ldv(T.s2, off + ic, body, R(1)) : R(1);
-    // horizontal: renormalised face values (:704-716, :1183-1193)
+    // horizontal: renormalised face values (:704-716, :1183-1193), three faces at a time:
+    // what they read of their neighbours first (six at once, or three in the 128 registers
+    // of four waves per SIMD, were slower: 0.49 and 0.62 against 0.39 ms)
     R fd = R(0);
-    for_slots(L.np, [&](int j) {
+    R s1nb[7], s2nb[7];
+    auto load = [&](auto j0, auto j1) {
+      constexpr int J0 = decltype(j0)::value, J1 = decltype(j1)::value;
+      if constexpr (!Q3) lim_nbr<J0, J1>(m, a, L, off, l, N);
+#pragma unroll
+      for (int j = J0; j < J1; ++j) {
+        const long nb = off + (long)L.nb[j] * ldk;
+        const R x1 = ldl(T.s1 + nb, (unsigned)l);
+        s1nb[j] = body ? x1 : R(1);
+        s2nb[j] = R(1);
+        if (mode == 1) {
+          const R x2 = ldl(T.s2 + nb, (unsigned)l);
+          s2nb[j] = body ? x2 : R(1);
+        }
+      }
+    };
+    auto face = [&](int j) {
       R low, hiv, sf, q0n;
-      lim_face(m, a, L, j, off, l, act, mode, qc, q0c, gxc, gyc, gqc, low, hiv, sf, q0n);
-      const long in = (long)L.nb[j] * ldk + l;
+      if constexpr (Q3) lim_face(m, a, L, j, off, l, act, mode, qc, q0c, gxc, gyc, gqc, low, hiv, sf, q0n);
+      else lim_face12(L, N, j, a.order, mode, qc, q0c, gxc, gyc, low, hiv, sf, q0n);
       const bool iw1side = L.dv[j] < R(0);
-      const R s1n = ldv(T.s1, off + in, body, R(1));
-      const R s2n = (mode == 1) ? ldv(T.s2, off + in, body, R(1)) : R(1);
+      const R s1n = s1nb[j], s2n = s2nb[j];
       const R s1_1 = iw1side ? s1c : s1n, s1_2 = iw1side ? s1n : s1c;
       const R s2_1 = iw1side ? s2c : s2n, s2_2 = iw1side ? s2n : s2c;
       R scale;
@@ -233,7 +305,21 @@ __global__ __launch_bounds__(256) void k_tr_lim_update(DMesh<R> m, TrStage<R, RP
       const R upv = low + hiv * scale;
       fd = fd + L.dv[j] * L.vm[j] * (upv - q0c);
       if (T.tsv && iw1side && body) T.tsv[n * T.vstride + (long)L.iv[j] * ldk + l] = scale;
-    });
+    };
+    using std::integral_constant;
+    constexpr int B = 3;
+    load(integral_constant<int, 0>{}, integral_constant<int, B>{});
+#pragma unroll
+    for (int j = 0; j < B; ++j) face(j);
+    if constexpr (B < 6) {
+      load(integral_constant<int, B>{}, integral_constant<int, 6>{});
+#pragma unroll
+      for (int j = B; j < 6; ++j) face(j);
+    }
+    if (L.np > 6) {
+      load(integral_constant<int, 6>{}, integral_constant<int, 7>{});
+      face(6);
+    }
     // vertical: renormalised fluxes (:1003-1008, :1396-1401)
     const R q0p1 = vshdn(m.tall, q0c, 1), qp1 = vshdn(m.tall, qc, 1);
     R upwl = (L.wm < R(0)) ? q0p1 : q0c;

@@ -839,7 +839,7 @@ struct Impl : ImplBase {
   std::vector<int> sgsmix;          // scalar_tab(n)%do_sgsmix, default .true. (var_tables.f90:59)
   DevBuf sgs_dev, rhof, lsct;       // do_sgsmix per tracer; nudged tracer density; adjoint of sct
   DevBuf lim_mode, lim_pre, lim_s1, lim_s2, lim_tsv, lim_tsw;
-  bool any_lim = false, any_pre = false, taped_lim = false;
+  bool any_lim = false, all_lim = false, any_pre = false, taped_lim = false;
   DevBuf ffimp, cflmax, nimp, anyimp, masspart, massout, mmkeys, mmout;
   // adjoint
   DevBuf adjA, adjB, lam0, nu, lpart, lgG, lgq[3];
@@ -1812,13 +1812,15 @@ struct Impl : ImplBase {
   // iscal_monot = 1, mode 2 with iscal_monot = 2 for pdef tracers, else 0 (regular
   // update); scp0 gets the low-order tendency update when iscal_monot > 0 and pdef.
   void lim_setup() {
-    any_lim = any_pre = false;
+    any_lim = all_lim = any_pre = false;
     if (prm.iscal_monot == 0 || ntr == 0) return;
     std::vector<int> mode(ntr), pre(ntr);
+    all_lim = true;
     for (int n = 0; n < ntr; ++n) {
       mode[n] = prm.iscal_monot == 1 ? 1 : (pdef[n] ? 2 : 0);
       pre[n] = pdef[n] ? 1 : 0;
       any_lim = any_lim || mode[n] != 0;
+      all_lim = all_lim && mode[n] != 0;
       any_pre = any_pre || (pre[n] && have_sct);
     }
     HIPCHK(hipMemcpyAsync(lim_mode.p, mode.data(), ntr * sizeof(int), hipMemcpyHostToDevice, s));
@@ -1878,8 +1880,8 @@ struct Impl : ImplBase {
         // two limiter passes
         const TrLim<R> L = lim_args(prm.adjoint_tape > 0);
         tracer_update(a);
-        LAUNCH("k_tr_lim_scales", (k_tr_lim_scales<R, RP>), dim3(nblk_tr()), dim3(256), dm, a, L);
-        LAUNCH("k_tr_lim_update", (k_tr_lim_update<R, RP>), dim3(nblk_tr()), dim3(256), dm, a, L);
+        if (dm.tall) a.order == 3 ? limited<true, true>(a, L) : limited<false, true>(a, L);
+        else a.order == 3 ? limited<true, false>(a, L) : limited<false, false>(a, L);
         taped_lim = prm.adjoint_tape > 0;
       } else if (use_patch && a.order < 3) {
         const dim3 g(pf.h.np), b(512);
@@ -1899,6 +1901,10 @@ struct Impl : ImplBase {
     have_fwd = true;
   }
 
+  template <bool Q3, bool TALL> void limited(const TrStage<R, RP> &a, const TrLim<R> &L) {
+    LAUNCH("k_tr_lim_scales", (k_tr_lim_scales<R, RP, Q3, TALL>), dim3(nblk_tr()), dim3(256), dm, a, L);
+    LAUNCH("k_tr_lim_update", (k_tr_lim_update<R, RP, Q3, TALL>), dim3(nblk_tr()), dim3(256), dm, a, L);
+  }
   // 16-byte pieces of the staged rows that a lane carries per tracer
   static constexpr int RING2_NCH = sizeof(R) == 4 ? 2 : 4;
   template <bool Q3, bool TALL> void ring2_fwd(const TrStage<R, RP> &a) {
@@ -1942,9 +1948,11 @@ struct Impl : ImplBase {
       const Q5<R> g{{(R *)a.gx, (R *)a.gy, dp<R>(trgq[0]), dp<R>(trgq[1]), dp<R>(trgq[2])}};
       LAUNCH("k_tr_grad3", (k_tr_grad3<R>), dim3(nblk_tr()), dim3(256), dm, a.q_in, g, ntr, tstride, tpw, a.tmode,
              a.lim);
+      if (a.lim && all_lim) return;             // no tracer left for the regular update
       if (dm.tall) LAUNCH("k_tr_update", (k_tr_update<R, RP, true, false, true>), dim3(nblk_tr()), dim3(256), dm, a);
       else LAUNCH("k_tr_update", (k_tr_update<R, RP, true>), dim3(nblk_tr()), dim3(256), dm, a);
     } else {
+      if (a.lim && all_lim) return;
       if (dm.tall) LAUNCH("k_tr_update", (k_tr_update<R, RP, false, false, true>), dim3(nblk_tr()), dim3(256), dm, a);
       else LAUNCH("k_tr_update", (k_tr_update<R, RP, false>), dim3(nblk_tr()), dim3(256), dm, a);
     }
@@ -2008,7 +2016,7 @@ struct Impl : ImplBase {
                sgs_dev.as<int>());
       if (a.lim) {
         const TrLim<R> L = lim_args(true);
-        adjoint_faces(a);
+        if (!all_lim) adjoint_faces(a);
         LAUNCH("k_tr_lim_adj0", (k_tr_lim_adj0<R, RP>), dim3(nblk_tr()), dim3(256), dm, a, L);
         LAUNCH("k_tr_lim_adj1", (k_tr_lim_adj1<R, RP>), dim3(nblk_tr()), dim3(256), dm, a, L);
         adjoint_coefs(a);
