@@ -694,10 +694,13 @@ __device__ __forceinline__ R vert_upw_monot(const DMesh<R> &m, R q, const R *scp
 // values of fluxes_wrtv's scalar_v_column (:1022-1081) and scalar_w_column.
 
 // The FP32 default instance is held to 64 VGPRs (8 waves per SIMD; a few spills, 3 %
-// faster at NXP=320, L=60); the other instances would spill far more under that bound.
+// faster at NXP=320, L=60) and the reference-precision one to 72 (7 waves instead of 6:
+// the acoustic step at NXP=160, L=50 7.64 -> 7.47 ms; 8 waves 8.09); the other instances
+// would spill far more.
 // Q3: some field has horizontal order 3 (the quadratic terms are only kept then).
 template <class R, class RP, bool MONO, bool NUD, bool Q3, bool TALL = false>
-__global__ __launch_bounds__(256, (sizeof(R) == 4 && sizeof(RP) == 4 && !MONO && !NUD && !Q3) ? OLAMGPU_BLOCKS_DYNW : 1)
+__global__ __launch_bounds__(256, (sizeof(R) == 4 && sizeof(RP) == 4 && !MONO && !NUD && !Q3) ? OLAMGPU_BLOCKS_DYNW
+                                 : (sizeof(R) == 4 && !MONO && !NUD && !Q3) ? 7 : 1)
 void k_dyn_w(DMesh<R> m, DynBuf<R, RP> b) {
   NOCONTRACT
   const WPos wp_ = wave_pos(TALL);
@@ -1140,10 +1143,14 @@ __global__ __launch_bounds__(256) void k_dyn_vn(DMesh<R> m, DynBuf<R, RP> b, int
 // vel_t3d.f90:39-108 (no closed faces on flat terrain).
 // N columns per wave (a wave pair for tall columns): the loads of all N columns are
 // issued before any is reduced.  Columns past the last one read the wave's first column
-// and store nothing.
-template <class R, class RP, int N>
+// and store nothing.  With the exchange code of tall columns out of the one-wave instance
+// one column a wave is as fast as eight on large meshes and faster on small ones (us per
+// launch, N = 1 / 8): 642 columns 6.6 / 9.9, 40,962 columns of 60 levels 26.5 / 28.8,
+// 256,002 145 / 145, 40,962 tall ones 45 / 48.
+template <class R, class RP, int N, bool TALL>
 __global__ __launch_bounds__(256) void k_dyn_veln(DMesh<R> m, DynBuf<R, RP> b) {
   NOCONTRACT
+  m.tall = TALL;          // known to the compiler: one-wave columns carry no exchange code
   const WPos p = wave_pos(m.tall);   // tall columns: the half from the wave index
   const int w = p.item;
   if (N * w >= m.nw) return;

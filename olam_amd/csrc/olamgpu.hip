@@ -30,7 +30,7 @@
 #define OLAMGPU_V_ITEMS 2
 #endif
 #ifndef OLAMGPU_VEL_ITEMS
-#define OLAMGPU_VEL_ITEMS 8
+#define OLAMGPU_VEL_ITEMS 1
 #endif
 #ifndef OLAMGPU_SETUPV_ITEMS
 #define OLAMGPU_SETUPV_ITEMS 2
@@ -1597,6 +1597,11 @@ struct Impl : ImplBase {
     }
   }
 
+  template <int N> void dyn_vel(const DynBuf<R, RP> &b) {
+    if (dm.tall) LAUNCH("k_dyn_vel", (k_dyn_veln<R, RP, N, true>), dim3(nblk_per(nw, N)), dim3(256), dm, b);
+    else LAUNCH("k_dyn_vel", (k_dyn_veln<R, RP, N, false>), dim3(nblk_per(nw, N)), dim3(256), dm, b);
+  }
+
   // rayf_init's copy of the initial wind (mem_rayf.f90:158-171); the profiles and b20
   // were built with the mesh
   void init_wrtv_rk() override {
@@ -1741,9 +1746,9 @@ struct Impl : ImplBase {
       }
       cur_thil = 1 - cur_thil;
       // several faces or columns per wave, their loads issued together
-      constexpr int NV = OLAMGPU_V_ITEMS, NVEL = OLAMGPU_VEL_ITEMS;
+      constexpr int NV = OLAMGPU_V_ITEMS;
       LAUNCH("k_dyn_v", (k_dyn_vn<R, RP, NV>), dim3(nblk_per(nv, NV)), dim3(256), dm, b, istage == nrk - 1 ? 1 : 0);
-      LAUNCH("k_dyn_vel", (k_dyn_veln<R, RP, NVEL>), dim3(nblk_per(nw, NVEL)), dim3(256), dm, b);
+      dyn_vel<OLAMGPU_VEL_ITEMS>(b);
     }
     HIPCHK(hipGetLastError());
   }
