@@ -46,6 +46,10 @@ struct DynBuf {
   int thil_order, wind_order, istage, nrk;
   double dt8;
   R fcor;
+  // sums of the horizontal advective fluxes formed by k_dyn_flux (FLUX instances of
+  // k_dyn_w): thil's here, the momenta's in vm[xyz]et_rk, the mass flux in press, which
+  // k_dyn_w then overwrites
+  const R *tt_flux;
 };
 
 // R-precision power evaluated through an FP64 pow and rounded once, so the FP32
@@ -698,7 +702,7 @@ __device__ __forceinline__ R vert_upw_monot(const DMesh<R> &m, R q, const R *scp
 // the acoustic step at NXP=160, L=50 7.64 -> 7.47 ms; 8 waves 8.09); the other instances
 // would spill far more.
 // Q3: some field has horizontal order 3 (the quadratic terms are only kept then).
-template <class R, class RP, bool MONO, bool NUD, bool Q3, bool TALL = false>
+template <class R, class RP, bool MONO, bool NUD, bool Q3, bool TALL = false, bool FLUX = false>
 __global__ __launch_bounds__(256, (sizeof(R) == 4 && sizeof(RP) == 4 && !MONO && !NUD && !Q3) ? OLAMGPU_BLOCKS_DYNW
                                  : (sizeof(R) == 4 && !MONO && !NUD && !Q3) ? 7 : 1)
 void k_dyn_w(DMesh<R> m, DynBuf<R, RP> b) {
@@ -724,15 +728,16 @@ void k_dyn_w(DMesh<R> m, DynBuf<R, RP> b) {
   R gqs[4][3] = {};
   for (int q = 0; q < 4; ++q) {
     const int ord = q == 0 ? b.thil_order : b.wind_order;
-    if (ord > 1) { gxs[q] = ld(b.g[2 * q], ic, act); gys[q] = ld(b.g[2 * q + 1], ic, act); }
+    if (!FLUX && ord > 1) { gxs[q] = ld(b.g[2 * q], ic, act); gys[q] = ld(b.g[2 * q + 1], ic, act); }
     if (Q3 && ord == 3)
       for (int t = 0; t < 3; ++t) gqs[q][t] = ld(b.gq[q][t], ic, act);
   }
   const R qc[4] = {thc, vxc, vyc, vzc};
   // horizontal advective fluxes (:632-661)
   RP hflx = RP(0);
-  R tt = ld_nt(b.thilt_s, ic, act), tx = ld_nt(b.vmxet_s, ic, act), ty = ld_nt(b.vmyet_s, ic, act),
-    tz = ld_nt(b.vmzet_s, ic, act);
+  R tt = ld_nt(FLUX ? b.tt_flux : b.thilt_s, ic, act), tx = ld_nt(FLUX ? b.vmxet_rk : b.vmxet_s, ic, act),
+    ty = ld_nt(FLUX ? b.vmyet_rk : b.vmyet_s, ic, act), tz = ld_nt(FLUX ? b.vmzet_rk : b.vmzet_s, ic, act);
+  if constexpr (FLUX) hflx = ld(b.press, ic, body);
   // nudging mass flux wmanud carrying the vertically upwinded values (:605-621,
   // nudflag == 1 with nud_preserve_total_mass), before the face sums
   if (NUD && b.nud_w) {
@@ -756,6 +761,7 @@ void k_dyn_w(DMesh<R> m, DynBuf<R, RP> b) {
       tz = tz + vz_m1 - vz;
     }
   }
+  if constexpr (!FLUX) {
   // face mass fluxes first: a neighbour's values and gradients are gathered only if some
   // level takes that face's value from the neighbour (upwind side)
   R vmca_j[7], vmc_j[7], arv_j[7];
@@ -851,6 +857,7 @@ void k_dyn_w(DMesh<R> m, DynBuf<R, RP> b) {
       tt = tt - vmca * f[0]; tx = tx - vmca * f[1]; ty = ty - vmca * f[2]; tz = tz - vmca * f[3];
     }
   });
+  }
   // Coriolis, global (:675-681)
   const RP rho_c = act ? b.rho[ic] : RP(0);
   const double vol = act ? m.volt[ic] : 0.0;

@@ -45,7 +45,8 @@ enum {
   R2_OUT = 48,                             // bit i set where outer face i's positive flux leaves n_j
   R2_NPOLY = 49,
   R2_PLACE = 50, R2_PLACEA = 55,           // places of the 18 cells and the column among its block's rows, bytes
-  R2_INTS = 60,
+  R2_GRAD = 60,                            // places of n_0..n_5 and the column among the block's gradients, bytes
+  R2_INTS = 62,
   // forward constants: dirv, then off and cof (nq terms x 6), then kf, per slot j {sum, prev,
   // next, mid_j-1, mid_j, far_j}
   R2_DIRV = 0, R2_OFF = 6,
@@ -610,6 +611,142 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
     ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
     if (more) {
       st_.put(smem_raw + ((n + 1 - ti.n0) & 1) * sg.bytes);
+      __syncthreads();
+    }
+  }
+}
+
+// ---------------------------------------------------------------- dynamics
+// The horizontal advective fluxes of prog_wrt_begs (prog_wrtv_rk.f90:632-661) with their
+// face values (fluxes_wrtv, :1022-1081) and gradients (grad_t2d), order 2, no nudging and
+// no monotone fluxes, columns of one wave: sums over the faces of mass, thil and the three
+// momenta, for k_dyn_w to finish the column with.  k_dyn_grad and the face loop of k_dyn_w,
+// which this replaces, wrote eight gradient fields and gathered twelve rows a face.  Per
+// field the block stages the rows of its columns' two rings (see Stager), forms the
+// gradients of its columns and their first ring, about 2.3 a column, in LDS, and each column
+// sums its faces from there.  The expressions and their order are those of k_dyn_grad and
+// k_dyn_w, so every sum is the same to the bit.
+// Entry e of a block's gradients belongs to wave e mod 16; a wave reads its up to four
+// entries at once, 16 lanes each, and broadcasts from there.
+// Bound by vector instructions (about 270 a column and field, four cycles each); ms a launch
+// of the gradient pass and the column kernel before, of this and the column kernel now:
+// 256,002 columns of 50 levels in mixed precision 0.29 + 1.10, 0.58 + 0.51; 1,024,002 of 60
+// in FP32 1.16 + 4.21, 2.36 + 1.94; 100,002 of 45 in FP64 0.27 + 0.77, 0.51 + 0.30.
+enum { R2_GWORDS = 16, R2_GENTRIES = WAVE / R2_GWORDS, R2_KD = 30 };
+template <class R>
+struct Ring2Grad {
+  const int *count;      // per block: cells whose gradient is formed
+  const int *place;      // per block and entry, 4 words: places of its slots 0..3 and 4..5, its own, 0 (bytes)
+  const R *cof;          // per block and entry, 16 words: gxps_coef, gyps_coef of its six slots
+  const R *kd;           // nw x R2_KD: dirv, dxps and dyps of this column's side, of the other side
+  int gmax;
+};
+template <class R, class RP>
+struct DynFlux {
+  const R *q[4];         // thil, vxe, vye, vze
+  const R *t[4];         // their volume-weighted tendencies, where the sums start
+  const R *vmc;
+  R *out[4];
+  RP *hflx;
+};
+template <class R, class RP, int NCH>
+__global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_dyn_flux(DMesh<R> m, Ring2Tab<R> t,
+                                                                                       Ring2Stage sg, Ring2Grad<R> gr,
+                                                                                       DynFlux<R, RP> a) {
+  NOCONTRACT
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int blk = xcd_block(blockIdx.x, gridDim.x), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = blk * RING2_NWF + wv, l = lane_id(), k = l + 1, mza = m.mza;
+  const bool own = w < m.nw;
+  const int c = min(w, m.nw - 1);
+  const bool body = k >= 2 && k <= mza;
+  const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
+                 mine = (unsigned)c * rowb, vb = (unsigned)m.nv * rowb;
+  unsigned char *grad = smem_raw + 2 * sg.bytes;
+  const RecI I(t.ints, c);
+  const RecK<R, R2_KD> K(gr.kd, c);
+  Stager<R, NCH, RING2_NWF> st(sg, blk, m.ldk);
+  st.get(Rows<R>(a.q[0], fb));
+  const int ng = gr.count[blk], mye = wv + (l / R2_GWORDS) * RING2_NWF;
+  R gk = R(0);
+  int gp = 0;
+  if (mye < ng) {
+    const long at = (long)blk * gr.gmax + mye;
+    gk = gr.cof[at * R2_GWORDS + l % R2_GWORDS];
+    gp = gr.place[at * 4 + l % 4];
+  }
+  // vmca = vmc * arv of the faces (:347-355)
+  R vm[6];
+  {
+    const Rows<R> v(a.vmc, vb), ar(m.arv, vb);
+    R x[6], y[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const unsigned f = (unsigned)I[R2_FACE + j] * rowb;
+      x[j] = v.get(lb, f);
+      y[j] = ar.get(lb, f);
+    }
+    const int np = I[R2_NPOLY];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) vm[j] = j < np ? x[j] * y[j] : R(0);
+  }
+  R tq = Rows<R>(a.t[0], fb).template get<ROWS_NT>(lb, mine);
+  st.put(smem_raw);
+  // slots in the order and with the signs of k_dyn_w: dirv > 0 adds
+  RP hflx = RP(0);
+#pragma unroll
+  for (int j = 0; j < 6; ++j) hflx = K[j] > R(0) ? hflx + (RP)vm[j] : hflx - (RP)vm[j];
+  if (own && body) a.hflx[(long)c * m.ldk + l] = hflx;
+  __syncthreads();
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+    unsigned char *buf = smem_raw + (q & 1) * sg.bytes;
+    R sum = tq;
+    if (q < 3) {
+      st.get(Rows<R>(a.q[q + 1], fb));
+      tq = Rows<R>(a.t[q + 1], fb).template get<ROWS_NT>(lb, mine);
+    }
+    // gradients (grad_t2d)
+#pragma unroll
+    for (int i = 0; i < R2_GENTRIES; ++i) {
+      const int e = wv + i * RING2_NWF, g0 = i * R2_GWORDS;
+      if (e >= ng) break;
+      const unsigned p03 = (unsigned)__builtin_amdgcn_readlane(gp, g0), p45 = (unsigned)__builtin_amdgcn_readlane(gp, g0 + 1),
+                     po = (unsigned)__builtin_amdgcn_readlane(gp, g0 + 2);
+      const R s0 = lds_row<R>(buf + lb, po * sg.pitch);
+      R ax = R(0), ay = R(0);
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        const unsigned place = ((j < 4 ? p03 : p45) >> (8 * (j & 3))) & 255u;
+        const R d = lds_row<R>(buf + lb, place * sg.pitch) - s0;
+        ax = ax + lane_word(gk, g0 + j) * d;
+        ay = ay + lane_word(gk, g0 + 6 + j) * d;
+      }
+      if (!body) { ax = R(0); ay = R(0); }
+      if (k <= mza) {
+        *reinterpret_cast<R *>(grad + (unsigned)(2 * e) * sg.pitch + lb) = ax;
+        *reinterpret_cast<R *>(grad + (unsigned)(2 * e + 1) * sg.pitch + lb) = ay;
+      }
+    }
+    __syncthreads();
+    auto place = [&](int i) { return (((unsigned)I[R2_PLACE + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch; };
+    auto gplace = [&](int i) { return (((unsigned)I[R2_GRAD + i / 4] >> (8 * (i % 4))) & 255u) * 2u * sg.pitch; };
+    const R qc = lds_row<R>(buf + lb, place(18));
+    const R gxs = lds_row<R>(grad + lb, gplace(6)), gys = lds_row<R>(grad + lb, gplace(6) + sg.pitch);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const R dv = K[j];
+      const R qn = lds_row<R>(buf + lb, place(j));
+      const R gxn = lds_row<R>(grad + lb, gplace(j)), gyn = lds_row<R>(grad + lb, gplace(j) + sg.pitch);
+      const R fs = qc + K[6 + j] * gxs + K[12 + j] * gys;
+      const R fn = qn + K[18 + j] * gxn + K[24 + j] * gyn;
+      const bool sel = (dv < R(0)) ? (vm[j] < R(0)) : !(vm[j] < R(0));
+      const R f = sel ? fn : fs;
+      sum = dv > R(0) ? sum + vm[j] * f : sum - vm[j] * f;
+    }
+    if (own && body) a.out[q][(long)c * m.ldk + l] = sum;
+    if (q < 3) {
+      st.put(smem_raw + ((q + 1) & 1) * sg.bytes);
       __syncthreads();
     }
   }

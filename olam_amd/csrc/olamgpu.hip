@@ -800,6 +800,11 @@ struct Impl : ImplBase {
   bool r2_stagef = false, r2_stagea = false;     // rows staged in LDS, forward and adjoint
   DevBuf b_r2n[2], b_r2cells[2];
   Ring2Stage r2f{}, r2a{};
+  bool use_flux = false;                         // k_dyn_flux
+  static constexpr int DYN_FLUX_NW = 2 * 256 * RING2_NWF;
+  unsigned flux_lds = 0;
+  DevBuf b_r2gn, b_r2gplace, b_r2gcof, b_r2kd;
+  Ring2Grad<R> r2g{};
   // state
   DevBuf thil[2], wmc, wc, vxe, vye, vze, vmc, vc, vmasc, wmasc, alpha, pwfac, pvfac, thilt, vmxet, vmyet, vmzet, vmt;
   DevBuf rho, press, rho_old;
@@ -909,7 +914,16 @@ struct Impl : ImplBase {
     if (use_patch) build_patch_tables();
     use_ring2 = prm.scal_horiz_adv_order >= 2 && ntr > 0 && !(use_patch || two_pass || fused_fwd || !fuse_adj) &&
                 mza <= RING2_TALL_MZA && std::max(wsz, vsz) * sizeof(R) < (size_t(1) << 32);
-    if (use_ring2) build_ring2_tables(m);
+    // the dynamics' flux sums from staged rows (k_dyn_flux): both fields at order 2, no
+    // nudging, fields below 4 GiB, columns of one wave and two blocks of 16 columns for each
+    // of 256 CUs; the stages with monotone fluxes keep the gradient pass.  us per acoustic
+    // step without / with it: 6,252 columns of 50 levels 338 / 343, 10,242 443 / 435, 16,002
+    // of 45 543 / 527 (FP64 910 / 818), 40,962 of 63 1218 / 1147, 256,002 of 50 (mixed) 7421 /
+    // 6593, 1,024,002 of 60 28273 / 25192.  Tall columns stage twice the rows for 16 waves: 40,962 of 100
+    // levels 2344 / 2720.
+    use_flux = prm.thil_horiz_adv_order == 2 && prm.wind_horiz_adv_order == 2 && prm.nudflag <= 0 && halves == 1 &&
+               nw >= DYN_FLUX_NW && std::max(wsz, vsz) * sizeof(R) < (size_t(1) << 32);
+    if (use_ring2 || use_flux) build_ring2_tables(m);
   }
 
   // Mesh constants of the two-ring stencil: with off_t(m, i) the reconstruction offsets of
@@ -919,8 +933,8 @@ struct Impl : ImplBase {
   // face i with sum_t cof_t(m, back) off_t(m, i) (ka).
   void build_ring2_tables(const olamgpu_mesh *m) {
     const Ring2 h = build_ring2(t, m);
-    if (!h.ok) { use_ring2 = false; return; }
-    const bool q3 = prm.scal_horiz_adv_order == 3;
+    if (!h.ok) { use_ring2 = use_flux = false; return; }
+    const bool q3 = use_ring2 && prm.scal_horiz_adv_order == 3;
     const int nt = q3 ? 5 : 2;
     In in{m};
     const float *offs[5] = {m->v_dxps, m->v_dyps, m->xx0_v, m->xy0_v, m->yy0_v};
@@ -935,19 +949,21 @@ struct Impl : ImplBase {
       for (int q = 0; q < nt; ++q) o[q] = offs[q][(size_t)(v + 1) * 2 + side];
     };
     const int nkf = r2_nkf(nt), KF = r2_kf(nt), COF = r2_cof(nt);
-    std::vector<R> kf((size_t)nw * nkf, R(0)), ka((size_t)nw * R2_NKA, R(0));
+    const size_t nk = use_ring2 ? nw : 0;            // k_dyn_flux reads the integers only
+    std::vector<R> kf(nk * nkf, R(0)), ka(nk * R2_NKA, R(0));
     std::vector<int> ints((size_t)nw * R2_INTS, 0);
     parallel_ranges(nw, [&](int c0, int c1) {
       for (int c = c0; c < c1; ++c) {
         const int np = t.w_npoly[c];
         int *I = &ints[(size_t)c * R2_INTS];
-        R *F = &kf[(size_t)c * nkf], *A = &ka[(size_t)c * R2_NKA];
         std::copy_n(&t.w_nbr[(size_t)c * NSLOT], 6, I + R2_NBR);
         std::copy_n(&h.cell[(size_t)c * 12], 12, I + R2_CELL);
         std::copy_n(&t.w_face[(size_t)c * NSLOT], 6, I + R2_FACE);
         std::copy_n(&h.face[(size_t)c * 24], 24, I + R2_OUTER);
         I[R2_OUT] = (int)h.out[c];
         I[R2_NPOLY] = np;
+        if (!use_ring2) continue;
+        R *F = &kf[(size_t)c * nkf], *A = &ka[(size_t)c * R2_NKA];
         double cs[5] = {};
         for (int j = 0; j < np; ++j) {
           double x[5], o[5];
@@ -989,13 +1005,86 @@ struct Impl : ImplBase {
     // 1 tracer 218 / 216 and 326 / 288, 2 tracers 259 / 280 and 367 / 379, 10 tracers 662 /
     // 926 and 890 / 1147; 10 tracers, 30 levels: 1,442 columns 15.1 / 14.1 and 15.5 / 14.9,
     // 5,762 columns 21.9 / 26.7 and 22.0 / 29.7.
-    if (std::min(ntr, tpw) >= 2 && nw >= 4096) {
-      r2_stagef = build_ring2_stage(ints, RING2_NWF, R2_PLACE, b_r2n[0], b_r2cells[0], r2f);
+    const bool many = use_ring2 && std::min(ntr, tpw) >= 2 && nw >= 4096;
+    if (many || use_flux) r2_stagef = build_ring2_stage(ints, RING2_NWF, R2_PLACE, b_r2n[0], b_r2cells[0], r2f);
+    use_flux = use_flux && r2_stagef && build_ring2_grad(m, ints);
+    r2_stagef = r2_stagef && many;
+    if (many) {
       r2_stagea = build_ring2_stage(ints, RING2_NWA, R2_PLACEA, b_r2n[1], b_r2cells[1], r2a);
     }
-    upv(b_r2ints, ints); upv(b_r2kf, kf); upv(b_r2ka, ka);
+    upv(b_r2ints, ints);
+    if (use_ring2) { upv(b_r2kf, kf); upv(b_r2ka, ka); }
     r2.ints = dp<int>(b_r2ints); r2.kf = dp<R>(b_r2kf); r2.ka = dp<R>(b_r2ka);
   }
+  // The cells of each block of k_dyn_flux whose gradient its columns read, and the places of
+  // their neighbours among the block's rows.  False where rows and gradients do not fit the
+  // LDS together.
+  bool build_ring2_grad(const olamgpu_mesh *m, std::vector<int> &ints) {
+    const int per = RING2_NWF, nb = (nw + per - 1) / per;
+    std::vector<int> list((size_t)nb * per * 7), cnt(nb, 0);
+    parallel_ranges(nb, [&](int b0, int b1) {
+      for (int b = b0; b < b1; ++b) {
+        int *r = &list[(size_t)b * per * 7], *e = r;
+        const int c1 = std::min(nw, (b + 1) * per);
+        for (int c = b * per; c < c1; ++c) {
+          *e++ = c;
+          e = std::copy_n(&ints[(size_t)c * R2_INTS + R2_NBR], 6, e);
+        }
+        std::sort(r, e);
+        cnt[b] = (int)(std::unique(r, e) - r);
+      }
+    });
+    const int gmax = *std::max_element(cnt.begin(), cnt.end());
+    flux_lds = 2 * r2f.bytes + ((unsigned)(2 * gmax) * r2f.pitch + (unsigned)(ldk * sizeof(R)) + 15) / 16 * 16;
+    int dev = 0, v = 0;
+    HIPCHK(hipGetDevice(&dev));
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0) v = 65536;
+    if (gmax > R2_GENTRIES * per || flux_lds > (unsigned)v) return false;
+    std::vector<int> rows((size_t)nb * r2f.nmax), rcnt(nb), where((size_t)nb * gmax * 4, 0);
+    std::vector<R> cof((size_t)nb * gmax * R2_GWORDS, R(0)), kd((size_t)nw * R2_KD, R(0));
+    HIPCHK(hipMemcpyAsync(rows.data(), b_r2cells[0].p, rows.size() * sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(rcnt.data(), b_r2n[0].p, rcnt.size() * sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    In in{m};
+    parallel_ranges(nb, [&](int b0, int b1) {
+      for (int b = b0; b < b1; ++b) {
+        const int *g = &list[(size_t)b * per * 7], *ge = g + cnt[b];
+        const int *r = &rows[(size_t)b * r2f.nmax], *re = r + rcnt[b];
+        auto place = [&](int x) { return (int)(std::lower_bound(r, re, x) - r) & 255; };
+        for (int i = 0; i < cnt[b]; ++i) {
+          int *o = &where[((size_t)b * gmax + i) * 4];
+          R *k = &cof[((size_t)b * gmax + i) * R2_GWORDS];
+          for (int j = 0; j < 6; ++j) o[j / 4] |= place(t.w_nbr[(size_t)g[i] * NSLOT + j]) << (8 * (j % 4));
+          o[2] = place(g[i]);
+          for (int j = 0; j < t.w_npoly[g[i]]; ++j) {
+            const size_t x = (size_t)(t.perm_w[g[i]] + 1) * 7 + j;
+            k[j] = (R)m->gxps_coef[x];
+            k[6 + j] = (R)m->gyps_coef[x];
+          }
+        }
+        const int c1 = std::min(nw, (b + 1) * per);
+        for (int c = b * per; c < c1; ++c) {
+          int *I = &ints[(size_t)c * R2_INTS];
+          for (int i = 0; i < 7; ++i)
+            I[R2_GRAD + i / 4] |= (int)(((unsigned)(std::lower_bound(g, ge, i < 6 ? I[i] : c) - g) & 255u) << (8 * (i % 4)));
+          R *k = &kd[(size_t)c * R2_KD];
+          for (int j = 0; j < t.w_npoly[c]; ++j) {
+            const int o = t.perm_w[c], v = in.iv(j, o);
+            const float dv = m->w_dirv[(size_t)(o + 1) * 7 + j];
+            const size_t own = (size_t)(v + 1) * 2 + (dv < 0.f ? 0 : 1), far = (size_t)(v + 1) * 2 + (dv < 0.f ? 1 : 0);
+            k[j] = (R)dv;
+            k[6 + j] = (R)m->v_dxps[own]; k[12 + j] = (R)m->v_dyps[own];
+            k[18 + j] = (R)m->v_dxps[far]; k[24 + j] = (R)m->v_dyps[far];
+          }
+        }
+      }
+    });
+    upv(b_r2gn, cnt); upv(b_r2gplace, where); upv(b_r2gcof, cof); upv(b_r2kd, kd);
+    r2g.place = dp<int>(b_r2gplace); r2g.cof = dp<R>(b_r2gcof); r2g.kd = dp<R>(b_r2kd);
+    r2g.count = dp<int>(b_r2gn); r2g.gmax = gmax;
+    return true;
+  }
+
   // Row lists of the staged blocks of nwv waves: the columns of a block and of their
   // rings, ascending, and at word `place` of each column's record the places of its cells
   // in that list.  False where the rows of some block do not fit the kernel's registers or
@@ -1708,7 +1797,18 @@ struct Impl : ImplBase {
       b.nud_rho = prm.nudflag > 0 && !prm.nud_preserve_total_mass;
       const bool nud = b.nud_vm || b.nud_w || b.nud_rho;
       int dth = prm.thil_horiz_adv_order == 2, dwn = prm.wind_horiz_adv_order == 2;
-      if (dth || dwn)
+      const bool flux = use_flux && !(istage == nrk && (mono_on[0] || mono_on[1]));
+      if (flux) {
+        DynFlux<R, RP> f;
+        const R *q[4] = {b.thil_in, b.vxe, b.vye, b.vze}, *ts[4] = {b.thilt_s, b.vmxet_s, b.vmyet_s, b.vmzet_s};
+        R *o[4] = {dp<R>(grads[0]), b.vmxet_rk, b.vmyet_rk, b.vmzet_rk};
+        for (int i = 0; i < 4; ++i) { f.q[i] = q[i]; f.t[i] = ts[i]; f.out[i] = o[i]; }
+        f.vmc = b.vmc;
+        f.hflx = b.press;
+        b.tt_flux = o[0];
+        LAUNCH_SH("k_dyn_flux", (k_dyn_flux<R, RP, RING2_NCH>), dim3((nw + RING2_NWF - 1u) / RING2_NWF),
+                  dim3(RING2_NWF * WAVE), flux_lds, dm, r2, r2f, r2g, f);
+      } else if (dth || dwn)
         LAUNCH("k_dyn_grad", (k_dyn_grad<R>), dim3(gw), dim3(256), dm, b.thil_in, b.vxe, b.vye, b.vze,
                            dp<R>(grads[0]), dp<R>(grads[1]), dp<R>(grads[2]), dp<R>(grads[3]), dp<R>(grads[4]),
                            dp<R>(grads[5]), dp<R>(grads[6]), dp<R>(grads[7]), dth, dwn);
@@ -1741,6 +1841,8 @@ struct Impl : ImplBase {
         LAUNCH("k_dyn_monot_pre", (k_dyn_monot_pre<R, RP>), dim3(gw), dim3(256), dm, mo, dp<RP>(rho0), (R)b.dt8);
         LAUNCH("k_dyn_monot_scales", (k_dyn_monot_scales<R, RP>), dim3(gw), dim3(256), dm, b, mo);
         launch_dyn_w<true>(b, nud, gw);
+      } else if (flux) {
+        LAUNCH("k_dyn_w", (k_dyn_w<R, RP, false, false, false, false, true>), dim3(gw), dim3(256), dm, b);
       } else {
         launch_dyn_w<false>(b, nud, gw);
       }
