@@ -628,10 +628,14 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
 // k_dyn_w, so every sum is the same to the bit.
 // Entry e of a block's gradients belongs to wave e mod 16; a wave reads its up to four
 // entries at once, 16 lanes each, and broadcasts from there.
-// Bound by vector instructions (about 270 a column and field, four cycles each); ms a launch
-// of the gradient pass and the column kernel before, of this and the column kernel now:
-// 256,002 columns of 50 levels in mixed precision 0.29 + 1.10, 0.58 + 0.51; 1,024,002 of 60
-// in FP32 1.16 + 4.21, 2.36 + 1.94; 100,002 of 45 in FP64 0.27 + 0.77, 0.51 + 0.30.
+// A face's upwind side, distances and places are the same for the four fields: they are
+// chosen once, per lane, and a field then costs one value, one gradient and six operations
+// a face (choosing per field: 256,002 columns 0.59 ms, now 0.50).  Bound by vector
+// instructions (about 180 a column and field, 1.2 of 2.0 ms at 1,024,002 columns) and the
+// bytes (4.7 GB, 0.9 ms there).  ms a launch of the gradient pass and the column kernel
+// before, of this and the column kernel now: 256,002 columns of 50 levels in mixed precision
+// 0.29 + 1.10, 0.50 + 0.51; 1,024,002 of 60 in FP32 1.16 + 4.21, 2.02 + 1.95; 100,002 of 45
+// in FP64 0.27 + 0.77, 0.41 + 0.29.
 enum { R2_GWORDS = 16, R2_GENTRIES = WAVE / R2_GWORDS, R2_KD = 30 };
 template <class R>
 struct Ring2Grad {
@@ -640,6 +644,10 @@ struct Ring2Grad {
   const R *cof;          // per block and entry, 16 words: gxps_coef, gyps_coef of its six slots
   const R *kd;           // nw x R2_KD: dirv, dxps and dyps of this column's side, of the other side
   int gmax;
+};
+template <class R>
+struct alignas(2 * sizeof(R)) GradPair {
+  R x, y;
 };
 template <class R, class RP>
 struct DynFlux {
@@ -676,7 +684,8 @@ __global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_dy
     gp = gr.place[at * 4 + l % 4];
   }
   // vmca = vmc * arv of the faces (:347-355)
-  R vm[6];
+  R vs[6], kx[6], ky[6];
+  unsigned qa[6], ga[6];
   {
     const Rows<R> v(a.vmc, vb), ar(m.arv, vb);
     R x[6], y[6];
@@ -688,25 +697,37 @@ __global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_dy
     }
     const int np = I[R2_NPOLY];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) vm[j] = j < np ? x[j] * y[j] : R(0);
+    for (int j = 0; j < 6; ++j) vs[j] = j < np ? x[j] * y[j] : R(0);
   }
   R tq = Rows<R>(a.t[0], fb).template get<ROWS_NT>(lb, mine);
   st.put(smem_raw);
-  // slots in the order and with the signs of k_dyn_w: dirv > 0 adds
+  // slots in the order and with the signs of k_dyn_w: dirv > 0 adds.  The upwind side, its
+  // distances and places are the same for every field.
   RP hflx = RP(0);
+  auto place = [&](int i) { return (((unsigned)I[R2_PLACE + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch; };
+  auto gplace = [&](int i) { return (((unsigned)I[R2_GRAD + i / 4] >> (8 * (i % 4))) & 255u) * 2u * sg.pitch; };
 #pragma unroll
-  for (int j = 0; j < 6; ++j) hflx = K[j] > R(0) ? hflx + (RP)vm[j] : hflx - (RP)vm[j];
+  for (int j = 0; j < 6; ++j) {
+    const R dv = K[j], vm = vs[j];
+    const bool sel = (dv < R(0)) ? (vm < R(0)) : !(vm < R(0));
+    hflx = dv > R(0) ? hflx + (RP)vm : hflx - (RP)vm;
+    vs[j] = dv > R(0) ? vm : -vm;
+    kx[j] = sel ? K[18 + j] : K[6 + j];
+    ky[j] = sel ? K[24 + j] : K[12 + j];
+    qa[j] = (sel ? place(j) : place(18)) + lb;
+    ga[j] = (sel ? gplace(j) : gplace(6)) + 2u * lb;
+  }
   if (own && body) a.hflx[(long)c * m.ldk + l] = hflx;
   __syncthreads();
 #pragma unroll 1
   for (int q = 0; q < 4; ++q) {
-    unsigned char *buf = smem_raw + (q & 1) * sg.bytes;
+    const unsigned char *buf = smem_raw + (q & 1) * sg.bytes;
     R sum = tq;
     if (q < 3) {
       st.get(Rows<R>(a.q[q + 1], fb));
       tq = Rows<R>(a.t[q + 1], fb).template get<ROWS_NT>(lb, mine);
     }
-    // gradients (grad_t2d)
+    // gradients (grad_t2d), x and y of a level side by side
 #pragma unroll
     for (int i = 0; i < R2_GENTRIES; ++i) {
       const int e = wv + i * RING2_NWF, g0 = i * R2_GWORDS;
@@ -717,32 +738,19 @@ __global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_dy
       R ax = R(0), ay = R(0);
 #pragma unroll
       for (int j = 0; j < 6; ++j) {
-        const unsigned place = ((j < 4 ? p03 : p45) >> (8 * (j & 3))) & 255u;
-        const R d = lds_row<R>(buf + lb, place * sg.pitch) - s0;
+        const R d = lds_row<R>(buf + lb, (((j < 4 ? p03 : p45) >> (8 * (j & 3))) & 255u) * sg.pitch) - s0;
         ax = ax + lane_word(gk, g0 + j) * d;
         ay = ay + lane_word(gk, g0 + 6 + j) * d;
       }
       if (!body) { ax = R(0); ay = R(0); }
-      if (k <= mza) {
-        *reinterpret_cast<R *>(grad + (unsigned)(2 * e) * sg.pitch + lb) = ax;
-        *reinterpret_cast<R *>(grad + (unsigned)(2 * e + 1) * sg.pitch + lb) = ay;
-      }
+      if (k <= mza) *reinterpret_cast<GradPair<R> *>(grad + (unsigned)e * 2u * sg.pitch + 2u * lb) = {ax, ay};
     }
     __syncthreads();
-    auto place = [&](int i) { return (((unsigned)I[R2_PLACE + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch; };
-    auto gplace = [&](int i) { return (((unsigned)I[R2_GRAD + i / 4] >> (8 * (i % 4))) & 255u) * 2u * sg.pitch; };
-    const R qc = lds_row<R>(buf + lb, place(18));
-    const R gxs = lds_row<R>(grad + lb, gplace(6)), gys = lds_row<R>(grad + lb, gplace(6) + sg.pitch);
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
-      const R dv = K[j];
-      const R qn = lds_row<R>(buf + lb, place(j));
-      const R gxn = lds_row<R>(grad + lb, gplace(j)), gyn = lds_row<R>(grad + lb, gplace(j) + sg.pitch);
-      const R fs = qc + K[6 + j] * gxs + K[12 + j] * gys;
-      const R fn = qn + K[18 + j] * gxn + K[24 + j] * gyn;
-      const bool sel = (dv < R(0)) ? (vm[j] < R(0)) : !(vm[j] < R(0));
-      const R f = sel ? fn : fs;
-      sum = dv > R(0) ? sum + vm[j] * f : sum - vm[j] * f;
+      const GradPair<R> g = *reinterpret_cast<const GradPair<R> *>(grad + ga[j]);
+      const R f = lds_row<R>(buf, qa[j]) + kx[j] * g.x + ky[j] * g.y;
+      sum = sum + vs[j] * f;
     }
     if (own && body) a.out[q][(long)c * m.ldk + l] = sum;
     if (q < 3) {

@@ -1035,7 +1035,7 @@ struct Impl : ImplBase {
       }
     });
     const int gmax = *std::max_element(cnt.begin(), cnt.end());
-    flux_lds = 2 * r2f.bytes + ((unsigned)(2 * gmax) * r2f.pitch + (unsigned)(ldk * sizeof(R)) + 15) / 16 * 16;
+    flux_lds = 2 * r2f.bytes + ((unsigned)(2 * gmax) * r2f.pitch + (unsigned)(2 * ldk * sizeof(R)) + 15) / 16 * 16;
     int dev = 0, v = 0;
     HIPCHK(hipGetDevice(&dev));
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0) v = 65536;
