@@ -63,6 +63,8 @@ def stage_alg_bytes(name, ntr, prec):
     per = {
         "k_tr_grad": tr, "k_tr_update": tr, "k_tr_stage": tr,
         "k_tr_adj0": tr, "k_tr_adj1": tr, "k_tr_adj01": tr, "k_tr_adj2": tr,
+        "k_tr_ring2": tr, "k_tr_ring2s": tr, "k_tr_ring2_adj": tr, "k_tr_ring2s_adj": tr,
+        "k_dyn_flux": 152 if mixed else 132,
         "k_dyn_w": 152 if mixed else 132,
         "k_dyn_v": 100 if mixed else 92,
         "k_dyn_vel": 28,
@@ -85,16 +87,20 @@ def kernel_alg_bytes(name, ntr, prec):
         "k_tr_adj01": 6 + 6 * ntr,            # vmasc, wmasc, volti, rho; mu, lam0 -> lam0, lpart, lgx, lgy
         "k_tr_adj2": 4 * ntr,                 # lpart, lgx, lgy -> lq
         "k_tr_stage": 6 + 3 * ntr,            # rho, volti, wmasc, vmasc; q, q0 -> q
-        # thil, vxe, vye, vze, their 8 gradients, 4 short-step tendencies, rho, volt (FP64),
-        # wmc, volti, alpha_press, rho0, rth0, pwfac, volwi, wmc0, wc, arw; vmc, arv on 3
-        # faces per cell -> press, rho, thil, vm[xyz]et_rk, wmc, wc
-        "k_dyn_w": 43,
+        "k_tr_ring2": 6 + 3 * ntr, "k_tr_ring2s": 6 + 3 * ntr,
+        # vr, wmasc, vmasc, rho; mu -> mu, and in one launch of three two earlier mu
+        "k_tr_ring2_adj": 6 + 8 * ntr / 3, "k_tr_ring2s_adj": 6 + 8 * ntr / 3,
+        # after k_dyn_flux: thil, vxe, vye, vze, the 4 sums and the mass sum, rho, volt (FP64),
+        # wmc, volti, alpha_press, rho0, rth0, pwfac, volwi, wmc0, wc, arw -> press, rho,
+        # thil, vm[xyz]et_rk, wmc, wc
+        "k_dyn_w": 30,
+        "k_dyn_flux": 19,                     # 4 fields, their tendencies; vmc, arv -> 5 sums
         "k_dyn_v": 23,                        # P2
         "k_dyn_vel": 7,                       # P3
     }.get(name)
     if per is None:
         return None
-    extra = {"k_dyn_w": 20, "k_dyn_v": 8}.get(name, 0) if prec == "mixed" else 0
+    extra = {"k_dyn_w": 24, "k_dyn_v": 8, "k_dyn_flux": 4}.get(name, 0) if prec == "mixed" else 0
     if prec == "f64" and name == "k_dyn_w":
         extra = -8                           # volt is one FP64 word, counted as two FP32 words
     return per * w + extra

@@ -3,7 +3,8 @@
 //
 // Reference: omodel/prog_wrtv_rk.f90, omodel/vort_div_damp.f90, omodel/vel_t3d.f90,
 // omodel/grad_lib.f90.  Per RK stage four launches replace the reference's ten
-// OpenMP loops: k_dyn_grad (grad_t2d of thil, vxe, vye, vze), k_dyn_w (fluxes_wrtv's
+// OpenMP loops: k_dyn_grad (grad_t2d of thil, vxe, vye, vze) or, on larger meshes,
+// k_dyn_flux of kernels_ring2.h (their face sums too), k_dyn_w (fluxes_wrtv's
 // face and vertical upwinding fused with prog_wrt_begs, including the FP64
 // tridiagonal W solve by parallel cyclic reduction inside the wavefront),
 // k_dyn_vn (prog_v_begs) and k_dyn_veln (vel_t3d_hex).

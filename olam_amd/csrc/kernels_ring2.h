@@ -1,5 +1,5 @@
 // kernels_ring2.h -- explicit tracer stages and their adjoint as one pass over the
-// two-ring stencil.
+// two-ring stencil, and the dynamics' flux sums from the same staged rows.
 //
 // With the winds given, an unlimited explicit stage is linear in the tracer, and its
 // weights do not depend on which tracer it is.  The face value of update_scalar
@@ -631,8 +631,8 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
 // A face's upwind side, distances and places are the same for the four fields: they are
 // chosen once, per lane, and a field then costs one value, one gradient and six operations
 // a face (choosing per field: 256,002 columns 0.59 ms, now 0.50).  Bound by vector
-// instructions (about 180 a column and field, 1.2 of 2.0 ms at 1,024,002 columns) and the
-// bytes (4.7 GB, 0.9 ms there).  ms a launch of the gradient pass and the column kernel
+// instructions (960 a column, 1.6 of 2.0 ms at 1,024,002 columns) and the bytes (5.8 GB, 1.0
+// ms there).  ms a launch of the gradient pass and the column kernel
 // before, of this and the column kernel now: 256,002 columns of 50 levels in mixed precision
 // 0.29 + 1.10, 0.50 + 0.51; 1,024,002 of 60 in FP32 1.16 + 4.21, 2.02 + 1.95; 100,002 of 45
 // in FP64 0.27 + 0.77, 0.41 + 0.29.

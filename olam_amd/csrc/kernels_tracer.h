@@ -1,7 +1,9 @@
 // kernels_tracer.h -- scalar_transport_rk (forward, adjoint) and its diagnostics.
 //
 // Reference: omodel/scalar_transport_rk.F90.  One wavefront per W column, lane l
-// holds level k = l+1.  The horizontal reconstruction is materialised per stage as
+// holds level k = l+1.  Unlimited stages of orders 2 and 3 and their adjoint run as one
+// pass over the two-ring stencil (kernels_ring2.h) where the mesh allows it.  The passes
+// here serve the other stages: the horizontal reconstruction is materialised per stage as
 // the gradient pair (gx, gy) of grad_t2d (grad_lib.f90:236-269), or at order 3 the five
 // terms of grad_t2d_quadratic (:278-341: gx, gy and the quadratic terms gq[0..2]); the
 // update kernel then rebuilds each V-face value from the upwind cell's coefficients,

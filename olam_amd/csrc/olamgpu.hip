@@ -917,10 +917,10 @@ struct Impl : ImplBase {
     // the dynamics' flux sums from staged rows (k_dyn_flux): both fields at order 2, no
     // nudging, fields below 4 GiB, columns of one wave and two blocks of 16 columns for each
     // of 256 CUs; the stages with monotone fluxes keep the gradient pass.  us per acoustic
-    // step without / with it: 6,252 columns of 50 levels 338 / 343, 10,242 443 / 435, 16,002
-    // of 45 543 / 527 (FP64 910 / 818), 40,962 of 63 1218 / 1147, 256,002 of 50 (mixed) 7421 /
-    // 6593, 1,024,002 of 60 28273 / 25192.  Tall columns stage twice the rows for 16 waves: 40,962 of 100
-    // levels 2344 / 2720.
+    // step without / with it: 4,412 columns of 50 levels 304 / 316, 6,252 340 / 340, 16,002 of
+    // 45 (mixed) 566 / 530, 40,962 of 50 1239 / 1112, 100,002 of 45 (FP64) 5115 / 4120, 256,002
+    // of 50 (mixed) 7421 / 6361, 1,024,002 of 60 28273 / 24092.  Tall columns stage twice the
+    // rows for 16 waves: 40,962 of 100 levels 2344 / 2720.
     use_flux = prm.thil_horiz_adv_order == 2 && prm.wind_horiz_adv_order == 2 && prm.nudflag <= 0 && halves == 1 &&
                nw >= DYN_FLUX_NW && std::max(wsz, vsz) * sizeof(R) < (size_t(1) << 32);
     if (use_ring2 || use_flux) build_ring2_tables(m);
