@@ -66,11 +66,18 @@ struct DevBuf {
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { if (p) (void)hipFree(p); }
-  void alloc(size_t b) {
-    if (p && bytes == b) return;                          // a new upload of the same size
-    if (p) { (void)hipFree(p); p = nullptr; }
+  // true where the memory is new; a buffer of that size stays, a failure leaves none, so a
+  // call that failed between its buffers is repeated by asking for all of them again
+  bool alloc(size_t b) {
+    if (p && bytes == b) return false;
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+    void *q = nullptr;
+    if (b) HIPCHK(hipMalloc(&q, b));
+    p = q;
     bytes = b;
-    if (b) HIPCHK(hipMalloc(&p, b));
+    return true;
   }
   template <class T> T *as() const { return (T *)p; }
 };
@@ -1502,15 +1509,22 @@ struct Impl : ImplBase {
     HIPCHK(hipStreamSynchronize(s));
   }
 
+  // allocated and cleared, or kept as it is
+  bool alloc_zero(DevBuf &b, size_t bytes) {
+    if (!b.alloc(bytes)) return false;
+    zero(b);
+    return true;
+  }
+
   void alloc_adj() {
-    if (adjA.p) return;
     size_t tb = std::max<size_t>(1, (size_t)ntr) * wsz * sizeof(R);
-    for (DevBuf *b : {&adjA, &adjB, &lam0, &nu, &lpart}) { b->alloc(tb); zero(*b); }
-    lgG.alloc(2 * tb); zero(lgG);
-    if (use_ring2) b_vr.alloc(wsz * sizeof(R));
+    bool any = false;
+    for (DevBuf *b : {&adjA, &adjB, &lam0, &nu, &lpart}) any |= alloc_zero(*b, tb);
+    any |= alloc_zero(lgG, 2 * tb);
+    if (use_ring2) any |= b_vr.alloc(wsz * sizeof(R));
     if (prm.scal_horiz_adv_order == 3)
-      for (DevBuf &b : lgq) { b.alloc(tb); zero(b); }
-    HIPCHK(hipStreamSynchronize(s));
+      for (DevBuf &b : lgq) any |= alloc_zero(b, tb);
+    if (any) HIPCHK(hipStreamSynchronize(s));
   }
 
   // -------------------------------------------------------------- transfers
@@ -1522,7 +1536,7 @@ struct Impl : ImplBase {
     const bool w = &perm == &t.perm_w;
     if (!w && &perm != &t.perm_v) throw Err(OLAMGPU_EINVAL, "transfer with an unknown numbering");
     DevBuf &p = w ? dperm_w : dperm_v, &q = w ? dinv_w : dinv_v;
-    if (!p.p) { upv(p, perm); upv(q, w ? t.inv_w : t.inv_v); }
+    if (!q.p) { upv(p, perm); upv(q, w ? t.inv_w : t.inv_v); }
     return (inverse ? q : p).as<int>();
   }
   template <class D, class H> void h2d_at(void *dst, const H *h, const std::vector<int> &perm) {
@@ -1617,15 +1631,16 @@ struct Impl : ImplBase {
   // -------------------------------------------------------------- prog_wrtv_rk
   // mem_nudge's wmanud, vmanud, rhot_nud (host Fortran layout; NULL keeps a field)
   void set_nudging(const float *wm, const float *vm, const double *rt) override {
-    if (!nud_w.p) alloc_nudging();
+    alloc_nudging();
     if (wm) h2d<R>(nud_w, wm, t.perm_w);
     if (vm) h2d<R>(nud_v, vm, t.perm_v);
     if (rt) h2d<RP>(nud_r, rt, t.perm_w);
   }
   void alloc_nudging() {
-    nud_w.alloc(wsz * sizeof(R)); nud_v.alloc(vsz * sizeof(R)); nud_r.alloc(wsz * sizeof(RP));
-    zero(nud_w); zero(nud_v); zero(nud_r);
-    HIPCHK(hipStreamSynchronize(s));
+    bool any = alloc_zero(nud_w, wsz * sizeof(R));
+    any |= alloc_zero(nud_v, vsz * sizeof(R));
+    any |= alloc_zero(nud_r, wsz * sizeof(RP));
+    if (any) HIPCHK(hipStreamSynchronize(s));
   }
 
   // the PBL scheme's mem_turb fields, then comp_horiz_k (pbl_driver.f90:136-238)
@@ -1642,11 +1657,9 @@ struct Impl : ImplBase {
       if (kh[c] < 0 || kh[c] > mza - 1 || km[c] < 0 || km[c] > mza - 1)
         throw Err(OLAMGPU_EINVAL, "khtop and kmtop must lie in [0, mza - 1]");
     }
-    if (!tb_vkh.p) {
-      tb_vkh.alloc(wsz * sizeof(R)); tb_vkm.alloc(wsz * sizeof(R));
-      tb_akhodx.alloc(vsz * sizeof(R)); tb_akmodx.alloc(vsz * sizeof(R));
-      tb_khtopv.alloc(nv * sizeof(int)); tb_kmtopv.alloc(nv * sizeof(int));
-    }
+    tb_vkh.alloc(wsz * sizeof(R)); tb_vkm.alloc(wsz * sizeof(R));
+    tb_akhodx.alloc(vsz * sizeof(R)); tb_akmodx.alloc(vsz * sizeof(R));
+    tb_khtopv.alloc(nv * sizeof(int)); tb_kmtopv.alloc(nv * sizeof(int));
     h2d<R>(tb_vkh, vkh, t.perm_w);
     h2d<R>(tb_vkm, vkm, t.perm_w);
     upv(tb_khtop, kh); upv(tb_kmtop, km); upv(tb_akm, as);
@@ -2384,10 +2397,12 @@ static int guarded(olamgpu_ctx *c, F &&f) {
     return OLAMGPU_OK;
   } catch (const Err &e) {
     if (c->impl) c->impl->drop_transfers();
+    (void)hipGetLastError();                  // or the next call's launches would report it
     c->err = e.what();
     return e.code;
   } catch (const std::exception &e) {
     if (c->impl) c->impl->drop_transfers();
+    (void)hipGetLastError();                  // or the next call's launches would report it
     c->err = e.what();
     return OLAMGPU_EHIP;
   }
@@ -2419,10 +2434,12 @@ int olamgpu_create(const olamgpu_mesh *mesh, const olamgpu_params *params, int32
       throw Err(OLAMGPU_EINVAL, "unknown precision mode");
   } catch (const Err &e) {
     g_err = e.what();
+    (void)hipGetLastError();
     olamgpu_destroy(c);
     return e.code;
   } catch (const std::exception &e) {
     g_err = e.what();
+    (void)hipGetLastError();
     olamgpu_destroy(c);
     return OLAMGPU_EHIP;
   }
