@@ -16,10 +16,10 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -154,7 +154,7 @@ struct CopyPool {
     th.reserve(n);
     try {
       while ((int)th.size() < n) th.emplace_back(&CopyPool::run, this, (int)th.size() + 1);
-    } catch (const std::system_error &) {                 // fewer threads than wished
+    } catch (const std::exception &) {                    // fewer threads than wished
     }
   }
   // one caller at a time (the context's)
@@ -557,7 +557,7 @@ template <class F> static void parallel_ranges(int n, F &&f) {
     const int b = std::min(n, a + part);
     try {
       th.emplace_back([&f, a, b] { f(a, b); });
-    } catch (const std::system_error &) {
+    } catch (const std::exception &) {                    // no thread, or no memory for one
       f(a, b);
     }
   }
@@ -2413,7 +2413,8 @@ extern "C" {
 int olamgpu_create(const olamgpu_mesh *mesh, const olamgpu_params *params, int32_t device, olamgpu_ctx **out) {
   if (!mesh || !params || !out) { g_err = "null argument"; return OLAMGPU_EINVAL; }
   *out = nullptr;
-  auto *c = new olamgpu_ctx;
+  auto *c = new (std::nothrow) olamgpu_ctx;
+  if (!c) return OLAMGPU_ENOMEM;
   try {
     int dev = device;
     if (dev < 0) HIPCHK(hipGetDevice(&dev));
