@@ -2192,24 +2192,25 @@ struct Impl : ImplBase {
   }
 
   // -------------------------------------------------------------- diagnostics
-  // per-block partial sums into part, then the sums of all blocks into out (device)
-  void mass_to(double *part, double *out) {
+  // per-block partial sums into part, then the sums of all blocks into out (device);
+  // prof is null for the caller that may take no event
+  void mass_to(double *part, double *out, Prof *prof) {
     const dim3 g(MASS_NB, (unsigned)std::max(1, (ntr + MASS_G - 1) / MASS_G));
     LAUNCH("k_mass_partial", (k_mass_partial<R, RP>), g, dim3(256), dm, dp<RP>(rho), dp<R>(trS), ntr, tstride, part);
     LAUNCH("k_mass_final", k_mass_final, dim3(1 + ntr), dim3(256), (const double *)part, MASS_NB, out);
     HIPCHK(hipGetLastError());
   }
   void mass_sums(double *out) override {
-    mass_to(masspart.as<double>(), massout.as<double>());
+    mass_to(masspart.as<double>(), massout.as<double>(), prof);
     HIPCHK(hipMemcpyAsync(out, massout.p, (1 + ntr) * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
   }
   // compute_mass_sums into a device array, with the partial sums in the static scratch
-  // (no allocation, no host copy)
+  // (no allocation, no event and no host copy, so its kernels are not timed)
   void mass_sums_noalloc(double *out_dev, double *scr) override {
     if (1 + ntr > MASS_NV) throw Err(OLAMGPU_EINVAL, "mass_sums_noalloc carries at most 64 tracers");
     if (!scr) throw Err(OLAMGPU_ESTATE, "scratch address not set up on this device");
-    mass_to(scr, out_dev);
+    mass_to(scr, out_dev, nullptr);
   }
   // tracer_maxmin (check_nans.F90:164-203): out[2n] = max, out[2n+1] = min of tracer n+1
   void tracer_maxmin(float *out) override {

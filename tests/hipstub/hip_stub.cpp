@@ -10,13 +10,14 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <vector>
 
 namespace {
 struct Dim { unsigned x, y, z; };
 std::mutex mu;
 std::map<const void *, std::string> &names() { static std::map<const void *, std::string> m; return m; }
-std::vector<std::string> &launched() { static std::vector<std::string> v; return v; }
+constexpr long LOG = 1 << 18;
+const char *launched[LOG];                         // takes no memory of the kind it counts
+long nlaunched = 0;
 long mallocs = 0, malloc_ok = -1, events = 0;      // malloc_ok: allocations that still succeed, -1 all
 int last = 0;
 std::atomic<long> news{0}, new_fail{0};            // the new_fail-th operator new from now on fails
@@ -40,8 +41,8 @@ long stub_events() { return events; }
 void stub_malloc_ok(long n) { malloc_ok = n; }
 long stub_news() { return news; }
 void stub_new_fail(long n) { new_fail = n; }
-long stub_launches() { return (long)launched().size(); }
-const char *stub_launch(long i) { return launched()[i].c_str(); }
+long stub_launches() { return nlaunched; }
+const char *stub_launch(long i) { return launched[i]; }
 
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
 void __hipUnregisterFatBinary(void **) {}
@@ -53,7 +54,9 @@ int __hipPushCallConfiguration(Dim g, Dim b, size_t sh, void *s) { cfg = {g, b, 
 int __hipPopCallConfiguration(Dim *g, Dim *b, size_t *sh, void **s) { *g = cfg.g; *b = cfg.b; *sh = cfg.sh; *s = cfg.s; return 0; }
 int hipLaunchKernel(const void *f, Dim, Dim, void **, size_t, void *) {
   std::lock_guard<std::mutex> l(mu);
-  launched().push_back(names()[f]);
+  const auto k = names().find(f);
+  if (nlaunched == LOG || k == names().end()) std::abort();
+  launched[nlaunched++] = k->second.c_str();
   return 0;
 }
 int hipGetLastError() { const int e = last; last = 0; return e; }
