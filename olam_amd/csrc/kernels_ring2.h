@@ -31,7 +31,14 @@
 // NXP=48, L=60, 8 tracers, order 3: 0.055 / 0.071 / 0.368 and 0.068 / 0.084 / 0.365 ms.
 // Over 40 steps of 8 FP32 tracers on 40,962 columns, <L q, lam> and <q, L^T lam> differ by
 // 2.1e-7 |q||lam| / sqrt(N) rms (4.9e-7 for the gradient and update passes).
-// A cell that is not finite makes its two rings not finite (its weight may be zero).
+// Zero weights and values that are not finite: 0 times such a value is not zero, so a sum over
+// all 18 cells would carry a NaN to both rings whatever the wind.  Where a sum comes out not
+// finite, it is formed again in those lanes without the cells and levels that the upwind side
+// does not read (skip), and the values that are not finite are those of the gradient and
+// update passes.  Where all is finite that costs one comparison a tracer: stages 0.5 to 1.5 %
+// longer forward, adjoint 1.3 % shorter (NXP=160, L=60, 10 tracers, fewer spilled scalars) to
+// 2.5 % longer (70 levels; one tracer).  Reading the fluxes again where it happens, instead of
+// keeping skip, was slower (gradient of 4 tracers at NXP=160 3.64 -> 3.90 ms).
 #pragma once
 #include "kernels_tracer.h"
 
@@ -91,6 +98,10 @@ struct RecK {
   }
   __device__ __forceinline__ R operator[](int i) const { return lane_word(v[i / WAVE], i % WAVE); }
 };
+
+// The word with the sign bit.
+__device__ __forceinline__ unsigned sign_word(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ unsigned sign_word(double v) { return (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32); }
 
 // shdn(v, 1) and shup(v, 1) with zero in the lane that has no source, in the form that the
 // compiler folds into the instruction using it.
@@ -212,6 +223,7 @@ __device__ __forceinline__ R lds_row(const unsigned char *buf, unsigned off) {
 template <class R>
 struct RingFwd {
   R C[18], S, v0, v1, v2, wf, vt, rinv;
+  unsigned skip;         // bit j: n_j is not upwind of face j; bit 6: the flux at this W level is not down
 };
 template <class R, class RP, bool Q3>
 __device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const RecK<R, r2_nkf(Q3 ? 5 : 2)> &K,
@@ -237,7 +249,8 @@ __device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const
   f.vt = Rows<R>(m.volti, fb).get(lb, own);
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
-    const R x = K[R2_DIRV + j] * vm[j];
+    const R x = K[R2_DIRV + j] * (vm[j] + R(0));        // -0 only where a face without flow is taken from here
+    f.skip = (j ? f.skip : 0u) | ((sign_word(x) >> (31 - j)) & (1u << j));
     w[j] = x > R(0) ? x : R(0);
     const R o = x - w[j];
     S = S + x;
@@ -255,6 +268,7 @@ __device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const
     f.C[12 + j] = w[j] * K[KF + 6 * j + 5];
   }
   if (I[R2_NPOLY] == 5) {         // n_4 and n_0 are neighbours; slot 5 reads the column itself
+    f.skip |= 1u << 5;
     f.C[0] = f.C[0] + w[4] * K[KF + 6 * 4 + 2];
     f.C[4] = f.C[4] + w[0] * K[KF + 1];
   }
@@ -264,27 +278,58 @@ __device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const
   f.wf = inner ? fexpl * wm : R(0);
   const int lp = min(l + 1, (int)ldk - 1);
   const bool neg = wm < R(0);
+  f.skip |= neg ? 0u : 64u;
   f.v0 = neg ? R(0) : f.wf * m.aw22[l];
   f.v1 = neg ? f.wf * (R(1) + m.aw21[lp]) : f.wf * m.aw12[l];
   f.v2 = neg ? f.wf * m.aw11[lp] : R(0);
   f.S = S + fexpl * (below0(wm) - wm);
   f.rinv = R(1) / (body ? rf : R(1));
 }
-// The new value from the column's value, scp0, tendency and the 18 cells' values; qn(i)
-// is called once per cell.
-template <class R, class F>
-__device__ __forceinline__ R ring_fwd_value(const RingFwd<R> &f, R qc, R q0, R st, R dtr, bool inner, int k, F &&qn) {
+// Keeps the rarely run second sum from sharing masks, addresses and loads with the first and
+// from loading ahead, which would hold registers throughout: v is new to the compiler, and
+// known only after `after`.
+template <class R>
+__device__ __forceinline__ void opaque(unsigned &v, R &after) {
+  asm volatile("" : "+v"(v), "+v"(after));
+}
+// The flux sum from the column's value, scp0 and the 18 cells' values; qn(i, 0) is called once
+// per cell.  GATED: only what the upwind side reads.
+template <bool GATED, class R, class F>
+__device__ __forceinline__ R ring_fwd_sum(const RingFwd<R> &f, R qc, R q0, bool inner, F &&qn) {
+  unsigned skip = f.skip, zero = 0u;
+  if constexpr (GATED) opaque(skip, qc);
+  auto unless = [&](unsigned bits, R v) { return GATED && (skip & bits) == bits ? R(0) : v; };
   R d = above0(qc) - qc;
   d = inner ? d : R(0);
-  const R y = f.v0 * below0(d) + f.v1 * d + f.v2 * above0(d);
+  const R da = unless(64u, above0(d)), dm = below0(d);      // moves with every lane, then chosen
+  const R db = GATED && !(skip & 64u) ? R(0) : dm;
+  const R y = f.v0 * db + f.v1 * d + f.v2 * da;
   const R x = y - f.wf * d;                     // the same flux against the level above
   R F0 = (qc - q0) * f.S + (below0(x) - y), F1 = R(0);
+  // ring 1 is always read: by the neighbour's own value or by this column's reconstruction
+  auto cells = [](int i) { return i < 6 ? ~0u : (1u << (i % 6)) | (i < 12 ? 1u << ((i + 1) % 6) : 0u); };
 #pragma unroll
   for (int i = 0; i < 18; i += 2) {
-    F0 = F0 + f.C[i] * (qn(i) - qc);
-    F1 = F1 + f.C[i + 1] * (qn(i + 1) - qc);
+    if constexpr (GATED) opaque(zero, F0);
+    F0 = F0 + f.C[i] * unless(cells(i), qn(i, zero) - qc);
+    F1 = F1 + f.C[i + 1] * unless(cells(i + 1), qn(i + 1, zero) - qc);
   }
-  F0 = F0 + F1;
+  return F0 + F1;
+}
+// true where a wave has to form its sum again
+template <class R>
+__device__ __forceinline__ bool any_not_finite(R v, bool where) {
+  return __builtin_expect(__ballot(where && !__builtin_isfinite(v)) != 0, 0);
+}
+// The new value from the column's value, scp0, tendency and the 18 cells' values.
+template <class R, class F>
+__device__ __forceinline__ R ring_fwd_value(const RingFwd<R> &f, R qc, R q0, R st, R dtr, bool inner, bool body, int k,
+                                            F &&qn) {
+  R F0 = ring_fwd_sum<false>(f, qc, q0, inner, qn);
+  if (any_not_finite(F0, body)) {
+    const R g = ring_fwd_sum<true>(f, qc, q0, inner, qn);
+    F0 = __builtin_isfinite(F0) ? F0 : g;
+  }
   R r = q0 + dtr * (st + f.vt * F0) * f.rinv;
   const R lev1 = above0(r);                     // level 1 copies level 2
   return k == 1 ? lev1 : r;
@@ -294,7 +339,7 @@ template <class R, class RP, bool Q3, bool TALL>
 __global__ __launch_bounds__(256) void k_tr_ring2(DMesh<R> m, Ring2Tab<R> t, TrStage<R, RP> a) {
   const RingItem ti = ring_item<TALL, WPB>(m.nw, a.ntr, a.tpw);
   const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
-  const bool inner = k >= 2 && k <= mza - 1;
+  const bool inner = k >= 2 && k <= mza - 1, body = k >= 2 && k <= mza;
   const long cb = (long)c * m.ldk;
   const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
                  own = (unsigned)c * rowb;
@@ -315,7 +360,7 @@ __global__ __launch_bounds__(256) void k_tr_ring2(DMesh<R> m, Ring2Tab<R> t, TrS
     for (int i = 0; i < 18; ++i) qn[i] = q.get(lb, row[i]);
     const R q0 = start ? qc : Rows<R>(a.q0 + fo, fb).template get<ROWS_NT>(lb, own);
     const R st = a.sct ? Rows<R>(a.sct + fo, fb).template get<ROWS_NT>(lb, own) : R(0);
-    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, k, [&](int i) { return qn[i]; });
+    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, body, k, [&](int i, unsigned) { return qn[i]; });
     if (k <= mza && ti.own) st_nt(a.q_out + fo, cb + l, r);
   }
 }
@@ -326,7 +371,7 @@ __global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_tr
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const RingItem ti = ring_item<TALL, RING2_NWF>(m.nw, a.ntr, a.tpw);
   const int c = ti.c, l = ti.l, k = l + 1, mza = m.mza;
-  const bool inner = k >= 2 && k <= mza - 1;
+  const bool inner = k >= 2 && k <= mza - 1, body = k >= 2 && k <= mza;
   const long cb = (long)c * m.ldk;
   const unsigned rowb = (unsigned)(m.ldk * sizeof(R)), fb = field_bytes(m), lb = (unsigned)l * (unsigned)sizeof(R),
                  own = (unsigned)c * rowb;
@@ -355,7 +400,8 @@ __global__ __launch_bounds__(RING2_NWF * WAVE, sizeof(R) == 4 ? 8 : 1) void k_tr
     const R q0 = start ? qc : q0n, st = stn;
     const bool more = n + 1 < ti.n1;
     if (more) fetch(n + 1);
-    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, k, [&](int i) { return lds_row<R>(buf, row[i]); });
+    const R r = ring_fwd_value(f, qc, q0, st, a.dtr, inner, body, k,
+                               [&](int i, unsigned z) { return lds_row<R>(buf, row[i] + z); });
     if (k <= mza && ti.own) st_nt(a.q_out + n * a.tstride, cb + l, r);
     if (more) {
       st_.put(smem_raw + ((n + 1 - ti.n0) & 1) * sg.bytes);
@@ -394,6 +440,7 @@ struct AdjHist {
 template <class R>
 struct RingAdj {
   R D[18], Dc, g, gc, cc, wf, al, be, cm, c0, cp;
+  unsigned skip;         // bit i: cell 6 + i is not read; bits 12, 13: the levels below (cm) and above (cp)
   bool rd0;
 };
 // vr(i): volti / rho of cell i (18: this column) at the lane's weight level
@@ -417,10 +464,12 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
   for (int i = 0; i < 24; ++i) vo[i] = vf.get(mb, (unsigned)I[R2_OUTER + i] * rowb);
   const unsigned out = (unsigned)I[R2_OUT];
 #pragma unroll
-  for (int i = 0; i < 24; ++i) vo[i] = vo[i] * (((out >> i) & 1u) ? R(1) : R(-1));     // outflow of n_j positive
+  for (int i = 0; i < 24; ++i)                  // outflow of n_j positive, -0 only where n_j does not give a face without flow its value
+    vo[i] = (vo[i] + R(0)) * (((out >> i) & 1u) ? R(1) : R(-1));
   const R wm = Rows<R>(a.wmasc, field_bytes(m)).get(lb, (unsigned)c * rowb);
   auto pos = [](R v) { return v > R(0) ? v : R(0); };
   R csum = R(0), fix0 = R(0), fix4 = R(0);
+  unsigned skip0 = 0u, skip1 = 0xfc0u;          // no flow from n_j to mid_j and far_j; from n_j+1 to mid_j
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     const int jm = (j + 5) % 6, jp = (j + 1) % 6;
@@ -440,12 +489,17 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
     D[6 + jm] = D[6 + jm] + tmp_;
     D[6 + j] = D[6 + j] + tmn;
     D[12 + j] = tf;
+    skip0 |= ((sign_word(vo[12 + j]) >> (31 - j)) & (1u << j)) | ((sign_word(vo[18 + j]) >> (25 - j)) & (64u << j));
+    skip1 |= (sign_word(vo[6 + j]) >> (31 - jm)) & (1u << jm);
   }
   if (I[R2_NPOLY] == 5) {         // n_4 and n_0 are neighbours, slot 5 is the column itself
+    skip0 |= 1u << 5;
+    skip1 |= 1u << 4;
     D[0] = D[0] + fix0;
     D[4] = D[4] + fix4;
     D[5] = R(0);
   }
+  f.skip = skip0 & skip1;
   // the weights of a column sum to zero; its own is summed ring by ring from the smallest
   // terms on (far, mid, ring 1), not one rounding after another at the size of the sum
   auto six = [&](int b) { return ((D[b] + D[b + 3]) + (D[b + 1] + D[b + 4])) + (D[b + 2] + D[b + 5]); };
@@ -466,9 +520,11 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
   const int lp = min(l + 1, (int)ldk - 1);
   f.al = (inner && !neg) ? R(1) : R(0);
   f.be = (body && k >= 3 && neg_m1) ? R(1) : R(0);
-  f.cm = (inner && k >= 3 && neg_m1) ? m.aw11[l] : R(0);
+  const bool below = inner && k >= 3 && neg_m1, above = k >= 2 && k <= mza - 2 && !neg_p1;
+  f.skip |= (below ? 0u : 1u << 12) | (above ? 0u : 1u << 13);
+  f.cm = below ? m.aw11[l] : R(0);
   f.c0 = inner ? (neg ? m.aw21[lp] : m.aw12[l]) : R(0);
-  f.cp = (k >= 2 && k <= mza - 2 && !neg_p1) ? m.aw22[lp] : R(0);
+  f.cp = above ? m.aw22[lp] : R(0);
   // on the first adjoint stage lam0 holds only what the implicit pass of this column wrote
   f.rd0 = !a.first || ff > R(0.001);
 }
@@ -478,26 +534,40 @@ __device__ __forceinline__ R ring_fold(R mr, bool body, int k) {
   const R below = below0(mr);
   return body ? (k == 2 ? mr + below : mr) : R(0);
 }
-// lq from the column's mu and its cells', and the stage's scp0 terms
+// lq from the column's mu (mr as read, nu of the stage) and its cells'; GATED as in
+// ring_fwd_sum
+template <bool GATED, class R, class F>
+__device__ __forceinline__ R ring_adj_sum(const RingAdj<R> &f, R mr, R nu, R dtr, int k, F &&mn) {
+  unsigned skip = f.skip, zero = 0u;
+  if constexpr (GATED) opaque(skip, nu);
+  auto unless = [&](unsigned bit, R v) { return GATED && (skip & bit) ? R(0) : v; };
+  const R L = f.wf * (above0(nu) - nu);
+  const R Lm = below0(L);
+  const R lds = f.cm * unless(1u << 12, Lm) + f.c0 * L + f.cp * unless(1u << 13, above0(L));
+  R acc = f.Dc * mr, acb = R(0);
+#pragma unroll
+  for (int i = 0; i < 18; i += 2) {
+    if constexpr (GATED) opaque(zero, acc);
+    acc = acc + f.D[i] * (i < 6 ? mn(i, zero) : unless(1u << (i - 6), mn(i, zero)));
+    acb = acb + f.D[i + 1] * (i < 6 ? mn(i + 1, zero) : unless(1u << (i - 5), mn(i + 1, zero)));
+  }
+  acc = acc + acb;
+  const R acc1 = below0(acc);
+  if (k == 2) acc = acc + acc1;
+  return dtr * acc + (f.al * L + f.be * Lm + (below0(lds) - lds));
+}
+// lq, and the stage's scp0 terms
 template <class R, class F>
 __device__ __forceinline__ R ring_adj_value(const RingAdj<R> &f, R mr, R &mu, R &nucc, R dtr, bool body, int k,
                                             F &&mn) {
   mu = ring_fold(mr, body, k);
   const R nu = mu * f.g;
   nucc = nu * f.cc;
-  const R L = f.wf * (above0(nu) - nu);
-  const R Lm = below0(L);
-  const R lds = f.cm * Lm + f.c0 * L + f.cp * above0(L);
-  R acc = f.Dc * mr, acb = R(0);
-#pragma unroll
-  for (int i = 0; i < 18; i += 2) {
-    acc = acc + f.D[i] * mn(i);
-    acb = acb + f.D[i + 1] * mn(i + 1);
+  R lq = ring_adj_sum<false>(f, mr, nu, dtr, k, mn);
+  if (any_not_finite(lq, body)) {
+    const R g = ring_adj_sum<true>(f, mr, nu, dtr, k, mn);
+    lq = __builtin_isfinite(lq) ? lq : g;
   }
-  acc = acc + acb;
-  const R acc1 = below0(acc);
-  if (k == 2) acc = acc + acc1;
-  const R lq = dtr * acc + (f.al * L + f.be * Lm + (below0(lds) - lds));
   return body ? lq : R(0);
 }
 
@@ -558,7 +628,7 @@ __global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t,
     const R p = p1 ? Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
     const R q2 = p2 ? Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
     R mu, nucc;
-    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i) { return mn[i]; });
+    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i, unsigned) { return mn[i]; });
     ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
   }
 }
@@ -607,7 +677,8 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
     const bool more = n + 1 < ti.n1;
     if (more) fetch(n + 1);
     R mu, nucc;
-    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i) { return lds_row<R>(buf, row[i]); });
+    const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k,
+                                 [&](int i, unsigned z) { return lds_row<R>(buf, row[i] + z); });
     ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
     if (more) {
       st_.put(smem_raw + ((n + 1 - ti.n0) & 1) * sg.bytes);
