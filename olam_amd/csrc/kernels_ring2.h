@@ -572,7 +572,9 @@ __device__ __forceinline__ R ring_adj_value(const RingAdj<R> &f, R mr, R &mu, R 
 }
 
 // The own-column rows a stage reads besides mu: lam0, or at the last stage of an AdjHist
-// the earlier stages' mu
+// the earlier stages' mu.  The stage writes over one of them, so a lane reads only what it
+// stores itself: not the levels that the other wave of a tall column stores, and nothing in a
+// wave past the last column.
 template <class R, class RP>
 __device__ __forceinline__ void ring_adj_rows(const TrAdj<R, RP> &a, const AdjHist<R> &h, bool rd0, const R *&p1,
                                               const R *&p2) {
@@ -625,8 +627,9 @@ __global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t,
     R mn[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) mn[i] = q.get(lb, row[i]);
-    const R p = p1 ? Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
-    const R q2 = p2 ? Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, row[18]) : R(0);
+    R p = R(0), q2 = R(0);
+    if (p1 && ti.own) p = Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, row[18]);
+    if (p2 && ti.own) q2 = Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, row[18]);
     R mu, nucc;
     const R lq = ring_adj_value(f, mr, mu, nucc, a.dtr, body, k, [&](int i, unsigned) { return mn[i]; });
     ring_adj_store(a, h, f, lq, mu, nucc, p, q2, body, k, act && ti.own, n, cb + l);
@@ -653,8 +656,8 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
   auto fetch = [&](int n) {
     const long fo = n * a.tstride;
     st_.get(Rows<R>(a.mu + fo, fb));
-    if (p1) pn = Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, own);
-    if (p2) qn = Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, own);
+    if (p1 && ti.own) pn = Rows<R>(p1 + fo, fb).template get<ROWS_NT>(lb, own);
+    if (p2 && ti.own) qn = Rows<R>(p2 + fo, fb).template get<ROWS_NT>(lb, own);
   };
   // vr goes where the second tracer will be; with it the first tracer, so that the
   // weights are formed with no rows in flight

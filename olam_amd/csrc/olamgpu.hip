@@ -2115,9 +2115,7 @@ struct Impl : ImplBase {
       LAUNCH("k_tr_vr", (k_tr_vr<R, RP>), dim3((unsigned)((wsz + 255) / 256)), dim3(256), dm, rho_tr, dp<R>(b_vr));
     // Two-ring stages without implicit columns keep mu of every stage: they go from the
     // current buffer X to the other (Y) and, in RK3, to lam0's (Z), and the last stage, which
-    // gathers from Y or Z and reads only its own columns of X and Y, writes X.  (The lanes of
-    // a tall column's wave that overlap the other wave may read what that one has written;
-    // they store nothing and no other lane uses their value.)
+    // gathers from Y or Z and reads of X and Y only what it stores itself, writes X.
     AdjHist<R> hist{};
     hist.on = use_ring2 && !any_imp && !any_lim;
     const DevBuf &hx = cur_adj_buf(), &hy = cur_adj ? adjA : adjB;
