@@ -107,22 +107,23 @@ __global__ __launch_bounds__(256) void k_pack(H *dst, const D *src, const int *i
   dst[i] = j == 0 ? H(0) : (H)src[(size_t)inv[j - 1] * ldk + l];
 }
 
-// Threads that share one host copy with the caller.  They belong to one context, start with
-// its first large transfer, wait between copies (a short spin, so that the chunks of one
-// transfer find them awake, then asleep) and end with the context.  Spawning them for each
-// chunk cost as much as a 10 MB copy.
+// Threads that share one host copy with the caller.  They belong to one context, are started
+// by the first copy that has a part for them, wait between copies (a short spin after a part,
+// so that the chunks of one transfer find them awake, then asleep) and end with the context.
+// The caller waits for the threads that have a part.  Spawning them for each chunk cost as
+// much as a 10 MB copy.
 struct CopyPool {
   static constexpr size_t PART = size_t(256) << 10;      // least bytes worth a thread
+  static constexpr unsigned long long PARTS = 16;        // job = copies so far * PARTS + parts of the last
   std::vector<std::thread> th;
   std::mutex mu;
   std::condition_variable cv;
-  std::atomic<unsigned> gen{0};
+  std::atomic<unsigned long long> job{0};
   std::atomic<int> left{0};
   std::atomic<bool> stop{false};
-  char *dst = nullptr;
+  char *dst = nullptr;                                    // read by the threads that have a part
   const char *src = nullptr;
   size_t part = 0, total = 0;
-  int parts = 1;
   ~CopyPool() {
     {
       std::lock_guard<std::mutex> lock(mu);
@@ -135,38 +136,42 @@ struct CopyPool {
     const size_t o = (size_t)k * part;
     if (o < total) std::memcpy(dst + o, src + o, std::min(part, total - o));
   }
-  void run(int k) {
-    unsigned seen = 0;
+  void run(int k, unsigned long long seen) {
+    bool spin = true;
     for (;;) {
-      for (int i = 0; i < 20000 && gen.load(std::memory_order_acquire) == seen && !stop; ++i) __builtin_ia32_pause();
-      if (gen.load(std::memory_order_acquire) == seen) {
+      for (int i = 0; spin && i < 20000 && job.load(std::memory_order_acquire) == seen && !stop; ++i)
+        __builtin_ia32_pause();
+      if (job.load(std::memory_order_acquire) == seen) {
         std::unique_lock<std::mutex> lock(mu);
-        cv.wait(lock, [&] { return gen.load(std::memory_order_acquire) != seen || stop; });
+        cv.wait(lock, [&] { return job.load(std::memory_order_acquire) != seen || stop; });
       }
       if (stop) return;
-      seen = gen.load(std::memory_order_acquire);
-      if (k < parts) slice(k);
+      seen = job.load(std::memory_order_acquire);
+      spin = k < (int)(seen % PARTS);
+      if (!spin) continue;
+      slice(k);
       left.fetch_sub(1, std::memory_order_release);
     }
   }
-  void start() {
-    const int n = (int)std::max(1u, std::min(8u, std::thread::hardware_concurrency())) - 1;
-    th.reserve(n);
+  void start(int n) {
     try {
-      while ((int)th.size() < n) th.emplace_back(&CopyPool::run, this, (int)th.size() + 1);
+      while ((int)th.size() < n) th.emplace_back(&CopyPool::run, this, (int)th.size() + 1, job.load());
     } catch (const std::exception &) {                    // fewer threads than wished
     }
   }
   // one caller at a time (the context's)
   void copy(void *d, const void *s, size_t nb) {
-    const int want = (int)std::min<size_t>(th.size() + 1, nb / PART);
+    const size_t most = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    const int wish = (int)std::min(most, nb / PART);
+    if (wish > 1) start(wish - 1);
+    const int want = std::min((int)th.size() + 1, wish);
     if (want < 2) { std::memcpy(d, s, nb); return; }
-    dst = (char *)d; src = (const char *)s; total = nb; parts = want;
+    dst = (char *)d; src = (const char *)s; total = nb;
     part = ((nb + want - 1) / want + 63) / 64 * 64;
-    left.store((int)th.size(), std::memory_order_relaxed);
+    left.store(want - 1, std::memory_order_relaxed);
     {
       std::lock_guard<std::mutex> lock(mu);
-      gen.fetch_add(1, std::memory_order_release);
+      job.store((job.load() / PARTS + 1) * PARTS + want, std::memory_order_release);
     }
     cv.notify_all();
     slice(0);
@@ -207,7 +212,6 @@ struct HostXfer {
         HIPCHK(hipEventRecord(ev[k], s));
       }
       have = want;
-      if (pool.th.empty()) pool.start();
     }
     // a larger staging buffer: what the stream still does with the old one comes first
     if (stage.bytes < bytes) {
