@@ -103,6 +103,11 @@ struct RecK {
 __device__ __forceinline__ unsigned sign_word(float v) { return __builtin_bit_cast(unsigned, v); }
 __device__ __forceinline__ unsigned sign_word(double v) { return (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32); }
 
+// v, and infinity for a NaN: a mass flux that is a NaN is not below zero, so its face takes the
+// value of the positive flux's side and must not count as one without flow.
+__device__ __forceinline__ float nan_up(float v) { return fminf(v, __builtin_inff()); }
+__device__ __forceinline__ double nan_up(double v) { return fmin(v, __builtin_inf()); }
+
 // shdn(v, 1) and shup(v, 1) with zero in the lane that has no source, in the form that the
 // compiler folds into the instruction using it.
 template <int CTRL>
@@ -465,7 +470,7 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
   const unsigned out = (unsigned)I[R2_OUT];
 #pragma unroll
   for (int i = 0; i < 24; ++i)                  // outflow of n_j positive, -0 only where n_j does not give a face without flow its value
-    vo[i] = (vo[i] + R(0)) * (((out >> i) & 1u) ? R(1) : R(-1));
+    vo[i] = nan_up(vo[i] + R(0)) * (((out >> i) & 1u) ? R(1) : R(-1));
   const R wm = Rows<R>(a.wmasc, field_bytes(m)).get(lb, (unsigned)c * rowb);
   auto pos = [](R v) { return v > R(0) ? v : R(0); };
   R csum = R(0), fix0 = R(0), fix4 = R(0);
@@ -506,6 +511,11 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
   const R Dc = -((six(12) + six(6)) + six(0));
 #pragma unroll
   for (int i = 0; i < 18; ++i) D[i] = D[i] * vr(i);
+  // a cell that is not read has no weight, whatever its density
+  if (any_not_finite((six(12) + six(6)), true)) {
+#pragma unroll
+    for (int i = 0; i < 12; ++i) D[6 + i] = (f.skip >> i) & 1u ? R(0) : D[6 + i];
+  }
   const R gc = vr(18);
   f.gc = body ? gc : R(0);
   f.g = a.dtr * f.gc;

@@ -1541,7 +1541,7 @@ __global__ void k_maxmin_init(int *keys, int n) {
 // One tracer per blockIdx.y; the waves of its blocks stride over the columns and keep the
 // extrema in registers, so a block ends in two atomics.  (Two atomics per column on the
 // 2 ntr keys serialised: 47.4 ms for 10 tracers of 256,002 columns and 50 levels; the
-// field's 0.84 GB now take 0.26 ms.)
+// 0.66 GB of padded columns now take 0.26 ms.)
 template <class R>
 __global__ __launch_bounds__(256) void k_tr_maxmin(DMesh<R> m, const R *q, long tstride, int *keys) {
   __shared__ float sh[WPB][2];

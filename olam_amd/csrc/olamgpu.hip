@@ -154,6 +154,7 @@ struct CopyPool {
     }
   }
   void start(int n) {
+    n = std::min(n, (int)std::thread::hardware_concurrency() - 1);
     try {
       while ((int)th.size() < n) th.emplace_back(&CopyPool::run, this, (int)th.size() + 1, job.load());
     } catch (const std::exception &) {                    // fewer threads than wished
@@ -161,9 +162,8 @@ struct CopyPool {
   }
   // one caller at a time (the context's)
   void copy(void *d, const void *s, size_t nb) {
-    const size_t most = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-    const int wish = (int)std::min(most, nb / PART);
-    if (wish > 1) start(wish - 1);
+    const int wish = (int)std::min<size_t>(8, nb / PART);
+    if (wish > (int)th.size() + 1) start(wish - 1);
     const int want = std::min((int)th.size() + 1, wish);
     if (want < 2) { std::memcpy(d, s, nb); return; }
     dst = (char *)d; src = (const char *)s; total = nb;
@@ -596,6 +596,9 @@ static Ring2 build_ring2(const Topo &t, const olamgpu_mesh *m) {
       int *cell = &r.cell[(size_t)c * 12], *face = &r.face[(size_t)c * 24], *slot = &r.slot[(size_t)c * 36];
       int rest[6][3], nrest[6];
       for (int i = 0; i < 12; ++i) cell[i] = c;
+      // absent faces have no weight and are faces of the column itself: one that is not finite
+      // reaches the column anyhow
+      for (int i = 0; i < 24; ++i) face[i] = t.w_face[(size_t)c * NSLOT];
       // the column's, the previous and the next ring-1 cell's slot in n_j, and the others
       for (int j = 0; j < np; ++j) {
         const int n = nb[j], prev = nb[(j + np - 1) % np], next = nb[(j + 1) % np];
@@ -979,7 +982,8 @@ struct Impl : ImplBase {
         int *I = &ints[(size_t)c * R2_INTS];
         std::copy_n(&t.w_nbr[(size_t)c * NSLOT], 6, I + R2_NBR);
         std::copy_n(&h.cell[(size_t)c * 12], 12, I + R2_CELL);
-        std::copy_n(&t.w_face[(size_t)c * NSLOT], 6, I + R2_FACE);
+        std::copy_n(&t.w_face[(size_t)c * NSLOT], np, I + R2_FACE);
+        if (np == 5) I[R2_FACE + 5] = I[R2_FACE];
         std::copy_n(&h.face[(size_t)c * 24], 24, I + R2_OUTER);
         I[R2_OUT] = (int)h.out[c];
         I[R2_NPOLY] = np;
