@@ -26,19 +26,22 @@
 // and run at the memory's rate per tracer plus the weights once per wave (about 240 and
 // 400 vector instructions).  Measured per stage, forward and adjoint, staged / gathered /
 // as gradient and update passes (k_tr_grad + k_tr_update, k_tr_adj01 + k_tr_adj2):
-// NXP=160, L=60, 10 tracers, FP32: 0.66 / 0.93 / 1.69 and 0.82 / 1.15 / 2.15 ms;
-// NXP=64, L=70, 20 tracers: 0.34 / 0.63 / 1.04 and 0.42 / 0.73 / 1.31 ms;
-// NXP=48, L=60, 8 tracers, order 3: 0.055 / 0.071 / 0.368 and 0.068 / 0.084 / 0.365 ms.
+// NXP=160, L=60, 10 tracers, FP32: 0.66 / 0.93 / 1.69 and 0.83 / 1.15 / 2.15 ms;
+// NXP=64, L=70, 20 tracers: 0.33 / 0.63 / 1.04 and 0.39 / 0.73 / 1.31 ms;
+// NXP=48, L=60, 8 tracers, order 3: 0.056 / 0.071 / 0.368 and 0.067 / 0.084 / 0.365 ms.
 // Over 40 steps of 8 FP32 tracers on 40,962 columns, <L q, lam> and <q, L^T lam> differ by
 // 2.1e-7 |q||lam| / sqrt(N) rms (4.9e-7 for the gradient and update passes).
 // Zero weights and values that are not finite: 0 times such a value is not zero, so a sum over
 // all 18 cells would carry a NaN to both rings whatever the wind.  Where a sum comes out not
 // finite, it is formed again in those lanes without the cells and levels that the upwind side
 // does not read (skip), and the values that are not finite are those of the gradient and
-// update passes.  Where all is finite that costs one comparison a tracer: stages 0.5 to 1.5 %
-// longer forward, adjoint 1.3 % shorter (NXP=160, L=60, 10 tracers, fewer spilled scalars) to
-// 2.5 % longer (70 levels; one tracer).  Reading the fluxes again where it happens, instead of
-// keeping skip, was slower (gradient of 4 tracers at NXP=160 3.64 -> 3.90 ms).
+// update passes, for tracers, adjoints, densities and fluxes.  Where all is finite that costs one
+// comparison a tracer and some 5 % more instructions for the weights, which the weights held as
+// formed (formed) give back.  Without / with it, forward and adjoint, us: NXP=160, L=60, 10
+// tracers 658 / 662 and 835 / 827; NXP=64, L=70, 20 tracers 327 / 329 and 410 / 388; one FP64
+// tracer at NXP=60, L=60 58.9 / 58.6 and 86.5 / 87.8; 8 FP32 tracers at NXP=16, L=60 14.9 / 15.6
+// and 16.2 / 16.7.  Reading the fluxes again where it happens, instead of keeping skip, was slower
+// (gradient of 4 tracers at NXP=160 3.64 -> 3.90 ms).
 #pragma once
 #include "kernels_tracer.h"
 
@@ -223,6 +226,14 @@ __device__ __forceinline__ R lds_row(const unsigned char *buf, unsigned off) {
   return *reinterpret_cast<const R *>(buf + off);
 }
 
+// The first N weights as formed: the compiler does not form them, or parts of them, again where
+// they are used, which spills scalar registers (k_tr_ring2 in FP64 40, none with it).
+template <int N, class R>
+__device__ __forceinline__ void formed(R *w) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(w[i]));
+}
+
 // Weights of one column for the forward stage (see the head of this file), and what the
 // vertical part and the update need of the column.
 template <class R>
@@ -277,6 +288,7 @@ __device__ __forceinline__ void ring_fwd(const DMesh<R> &m, const RecI &I, const
     f.C[0] = f.C[0] + w[4] * K[KF + 6 * 4 + 2];
     f.C[4] = f.C[4] + w[0] * K[KF + 1];
   }
+  formed<18>(f.C);
   // vertical: with d(k) = q(k+1) - q(k) on levels 2..mza-1 the upwinded value at W level k
   // less q(k) is v0 d(k-1) + v1 d(k) + v2 d(k+1) (grad_z_quadratic, bounded)
   const R fexpl = R(1) - a.ffimp[(long)(a.istage - 1) * m.nw + c];
@@ -448,8 +460,14 @@ struct RingAdj {
   unsigned skip;         // bit i: cell 6 + i is not read; bits 12, 13: the levels below (cm) and above (cp)
   bool rd0;
 };
-// vr(i): volti / rho of cell i (18: this column) at the lane's weight level
-template <class R, class RP, class F>
+// vr(i): volti / rho of cell i (18: this column) at the lane's weight level.
+// FORMED weights are held as formed (formed()): all, or those that leave k_tr_ring2_adj in FP64
+// its 4 waves per SIMD (12: 117 registers; 18: 135 and 3 waves; 60 levels, one tracer, order 2 at
+// NXP=60 87.6 us, 103 with 18 of them spilled to 128 registers).  0, the FP32 k_tr_ring2s_adj,
+// which a branch suits better (NXP=160, L=60, 10 tracers 827 us, 845 with 18; NXP=64, L=70, 20
+// tracers 388 and 411): one that sets the weights of cells that are not read to zero where a
+// density is not finite, as the gated sum does with their products.
+template <int FORMED, class R, class RP, class F>
 __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const RecK<R, R2_NKA> &K,
                                          const TrAdj<R, RP> &a, int c, int l, RingAdj<R> &f, F &&vr) {
   const int k = l + 1, mza = m.mza;
@@ -511,8 +529,9 @@ __device__ __forceinline__ void ring_adj(const DMesh<R> &m, const RecI &I, const
   const R Dc = -((six(12) + six(6)) + six(0));
 #pragma unroll
   for (int i = 0; i < 18; ++i) D[i] = D[i] * vr(i);
-  // a cell that is not read has no weight, whatever its density
-  if (any_not_finite((six(12) + six(6)), true)) {
+  if constexpr (FORMED > 0) {
+    formed<FORMED>(D);
+  } else if (any_not_finite((six(12) + six(6)), true)) {
 #pragma unroll
     for (int i = 0; i < 12; ++i) D[6 + i] = (f.skip >> i) & 1u ? R(0) : D[6 + i];
   }
@@ -558,8 +577,9 @@ __device__ __forceinline__ R ring_adj_sum(const RingAdj<R> &f, R mr, R nu, R dtr
 #pragma unroll
   for (int i = 0; i < 18; i += 2) {
     if constexpr (GATED) opaque(zero, acc);
-    acc = acc + f.D[i] * (i < 6 ? mn(i, zero) : unless(1u << (i - 6), mn(i, zero)));
-    acb = acb + f.D[i + 1] * (i < 6 ? mn(i + 1, zero) : unless(1u << (i - 5), mn(i + 1, zero)));
+    // the product: a cell that is not read has no weight, whatever its density
+    acc = acc + (i < 6 ? f.D[i] * mn(i, zero) : unless(1u << (i - 6), f.D[i] * mn(i, zero)));
+    acb = acb + (i < 6 ? f.D[i + 1] * mn(i + 1, zero) : unless(1u << (i - 5), f.D[i + 1] * mn(i + 1, zero)));
   }
   acc = acc + acb;
   const R acc1 = below0(acc);
@@ -627,7 +647,7 @@ __global__ __launch_bounds__(256) void k_tr_ring2_adj(DMesh<R> m, Ring2Tab<R> t,
   row[18] = (unsigned)c * rowb;
   const Rows<R> gr(vr, fb);
   RingAdj<R> f;
-  ring_adj(m, I, K, a, c, l, f, [&](int i) { return gr.get(mb, row[i]); });
+  ring_adj<sizeof(R) == 4 ? 18 : 12>(m, I, K, a, c, l, f, [&](int i) { return gr.get(mb, row[i]); });
   const R *p1, *p2;
   ring_adj_rows(a, h, f.rd0, p1, p2);
   for (int n = ti.n0; n < ti.n1; ++n) {
@@ -681,7 +701,8 @@ __global__ __launch_bounds__(RING2_NWA * WAVE, sizeof(R) == 4 ? 6 : 1) void k_tr
 #pragma unroll
   for (int i = 0; i < 19; ++i) row[i] = (((unsigned)I[R2_PLACEA + i / 4] >> (8 * (i % 4))) & 255u) * sg.pitch;
   RingAdj<R> f;
-  ring_adj(m, I, K, a, c, l, f, [&](int i) { return lds_row<R>(smem_raw + sg.bytes + mb, row[i]); });
+  ring_adj<sizeof(R) == 4 ? 0 : 18>(m, I, K, a, c, l, f,
+                                    [&](int i) { return lds_row<R>(smem_raw + sg.bytes + mb, row[i]); });
   __syncthreads();
   for (int n = ti.n0; n < ti.n1; ++n) {
     const unsigned char *buf = smem_raw + ((n - ti.n0) & 1) * sg.bytes + lb;
